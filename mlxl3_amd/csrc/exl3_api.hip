@@ -276,6 +276,7 @@ static constexpr int kTileCounters = 256;
 
 struct QmmShape {
   int mb, mtiles, splits;
+  double cost;  // modelled ns
 };
 
 static QmmShape choose_qmm_shape(int in, int out, int64_t rows) {
@@ -286,7 +287,7 @@ static QmmShape choose_qmm_shape(int in, int out, int64_t rows) {
     if (v == 1 || v == 2 || v == 4) force_mb = v;
   }
   if (const char* env = getenv("EXL3_QMM_SPLITS")) force_splits = std::max(0, atoi(env));
-  QmmShape best{4, (int)((rows + 255) / 256), 1};
+  QmmShape best{4, (int)((rows + 255) / 256), 1, 0};
   double best_cost = 1e300;
   for (int mb : {4, 2, 1}) {
     if (force_mb && mb != force_mb) continue;
@@ -302,7 +303,7 @@ static QmmShape choose_qmm_shape(int in, int out, int64_t rows) {
       if (s > 1) cost += 0.7 / 1024 * 4.0 * (double)s * mt * 64 * mb * out;
       if (cost < best_cost) {
         best_cost = cost;
-        best = QmmShape{mb, (int)mt, s};
+        best = QmmShape{mb, (int)mt, s, cost};
       }
       if (force_splits) break;
     }
@@ -315,6 +316,57 @@ static QmmShape choose_qmm_shape(int in, int out, int64_t rows) {
 static size_t qmm_partial_bytes(const QmmShape& sh, int out) {
   if (sh.splits <= 1) return 0;
   return sizeof(float) * (size_t)sh.splits * sh.mtiles * (out / 128) * 64 * sh.mb * 128;
+}
+
+// Launch shape of the decode-in-registers QMM (exl3_wide.hpp): 16*R rows x 256
+// columns per workgroup, one workgroup per CU at R = 8 and 16, two at R = 4.
+// Rounds of workgroups x (steps of 64 inputs per split) x the step time (ns,
+// every CU busy: R = 4 1500 with two workgroups, 8 1060, 16 1560), a fixed part
+// per launch (ring fill, epilogue, output flush: 8 / 9 / 15 us) and, with
+// splits, 3 us and 0.42 ns per KB of f32 partials for the summing launch.
+// Measured against the producer/consumer kernel on one box (us, the better shape
+// of each): 4096x28672 M 384/512/1024/2048 162/159/322/578 -> 120/126/246/494,
+// 14336x4096 M 256/512/1024/4096 61/98/160/567 -> 55/87/147/482, 27648x5120 M
+// 256/512/2048 116/196/939 -> 103/169/602, 5120x7168 M 384/2048 67/202 ->
+// 53/159; it loses on small launches (2048x1536 M 64..1024 16-32 -> 18-33,
+// 4096x4096 M 64/128 21/24 -> 24/28), where its 256-column tiles are too few.
+struct WideShape {
+  int r, mtiles, splits;
+  double cost;
+};
+
+static size_t wide_partial_bytes(int r, int mtiles, int pairs, int splits) {
+  return splits > 1 ? sizeof(float) * (size_t)splits * mtiles * pairs * 16 * r * 256 : 0;
+}
+
+// The cheapest shape whose partials fit in `budget` bytes (one split always fits).
+static WideShape choose_wide_shape(int in, int pairs, int64_t rows, size_t budget) {
+  const int nq = in / 64;
+  int force_r = 0, force_splits = 0;
+  if (const char* env = getenv("EXL3_WIDE_R")) force_r = atoi(env);
+  if (const char* env = getenv("EXL3_WIDE_SPLITS")) force_splits = std::max(0, atoi(env));
+  WideShape best{16, (int)((rows + 255) / 256), 1, 1e300};
+  for (int r : {4, 8, 16}) {
+    if (force_r && r != force_r) continue;
+    const int64_t mt = (rows + 16 * r - 1) / (16 * r);
+    const int per_round = r == 4 ? 512 : 256;
+    const double step_ns = r == 4 ? 1500.0 : r == 8 ? 1060.0 : 1560.0;
+    const double fixed = r == 4 ? 8000.0 : r == 8 ? 9000.0 : 15000.0;
+    for (int splits = 1; splits <= 8; ++splits) {
+      int sp = force_splits ? force_splits : splits;
+      sp = std::max(1, std::min(sp, std::max(1, nq / 4)));
+      const size_t part = wide_partial_bytes(r, (int)mt, pairs, sp);
+      if (part > budget) continue;
+      const int64_t wgs = mt * pairs * sp, rounds = (wgs + per_round - 1) / per_round;
+      // half-empty CUs of an R = 4 launch run their one workgroup faster
+      const double step = r == 4 && wgs <= 256 ? 900.0 : step_ns;
+      double cost = fixed + (double)rounds * ((nq + sp - 1) / sp) * step;
+      if (sp > 1) cost += 3000.0 + 0.42 / 1024 * (double)part;
+      if (cost < best.cost) best = WideShape{r, (int)mt, sp, cost};
+      if (force_splits) break;
+    }
+  }
+  return best;
 }
 
 // Workspace: the first kWorkspaceCounterBytes hold split-K counters that are
@@ -395,6 +447,51 @@ static bool qmv_fragment_exchange(int64_t rows, int kw) {
   return kw == 1 && rows >= from;
 }
 
+// Column pairs (256 columns) of a group: a member's last one may be half empty.
+static int group_pairs(const Group& g) {
+  int pairs = 0;
+  for (int i = 0; i < g.count; ++i) pairs += (g.parts[i]->out + 255) / 256;
+  return pairs;
+}
+
+// Whether a QMM over the group runs in registers (exl3_wide.hpp) and in which
+// shape, with `budget` bytes for partials: where it is modelled faster than the
+// producer/consumer kernel (whose model leaves out ~6 us of ring fill and
+// epilogue).  Its trellis copies are 16 bytes wide, so every trellis has to be
+// 16-byte aligned (a checkpoint's tensors are; a caller's view may not be).
+// EXL3_WIDE=0/1 forces it off or on (tuning).
+static bool group_takes_wide(const Group& g, int64_t rows, size_t budget, WideShape* shape) {
+  for (int i = 0; i < g.count; ++i)
+    if ((uintptr_t)g.parts[i]->trellis & 15) return false;
+  *shape = choose_wide_shape(g.in, group_pairs(g), rows, budget);
+  if (const char* env = getenv("EXL3_WIDE")) return atoi(env) != 0;
+  return shape->cost < choose_qmm_shape(g.in, g.total_out, rows).cost + 6000.0;
+}
+
+// Split-K partials of the producer/consumer QMM over the group: what every
+// workspace has to hold.
+static size_t group_qmm_partials_min(const Group& g, int64_t rows) {
+  return qmm_partial_bytes(choose_qmm_shape(g.in, g.total_out, rows), g.total_out);
+}
+// The partials a launch may choose: any amount, but where the allocation-free
+// entry point serves the call (one projection that fits its fixed workspace at
+// the least), no more than fits there, so both entry points run the same shape
+// and give the same bits.
+static size_t group_partial_budget(const Group& g, int64_t rows) {
+  if (g.count > 1) return SIZE_MAX;
+  const size_t room = kNoAllocBytes - kWorkspaceCounterBytes;
+  const size_t xhat = align_up(sizeof(uint16_t) * (size_t)rows * g.in);
+  return xhat + align_up(group_qmm_partials_min(g, rows)) > room ? SIZE_MAX : room - xhat;
+}
+// ... and what the launch takes when it is given: a workspace between the two
+// gets the fastest shape that fits.
+static size_t group_qmm_partials(const Group& g, int64_t rows) {
+  WideShape sh;
+  const size_t least = group_qmm_partials_min(g, rows);
+  if (!group_takes_wide(g, rows, group_partial_budget(g, rows), &sh)) return least;
+  return std::max(least, wide_partial_bytes(sh.r, sh.mtiles, group_pairs(g), sh.splits));
+}
+
 // Scratch bytes (after the counter region) of one group launch.
 static size_t group_scratch_bytes(const Group& g, int64_t rows) {
   if (rows <= kQmvMaxRows) {
@@ -410,9 +507,15 @@ static size_t group_scratch_bytes(const Group& g, int64_t rows) {
                                 : sizeof(float) * (size_t)splits * rows * g.total_out;
     return xhat + align_up(partials);
   }
-  const QmmShape sh = choose_qmm_shape(g.in, g.total_out, rows);
-  const size_t partials = qmm_partial_bytes(sh, g.total_out);
-  return (size_t)g.count * align_up(sizeof(uint16_t) * (size_t)rows * g.in) + align_up(partials);
+  return (size_t)g.count * align_up(sizeof(uint16_t) * (size_t)rows * g.in) +
+         align_up(group_qmm_partials(g, rows));
+}
+
+// ... that a call cannot do without.
+static size_t group_scratch_min(const Group& g, int64_t rows) {
+  if (rows <= kQmvMaxRows) return group_scratch_bytes(g, rows);
+  return (size_t)g.count * align_up(sizeof(uint16_t) * (size_t)rows * g.in) +
+         align_up(group_qmm_partials_min(g, rows));
 }
 
 static int check_rows(const Group& g, int64_t rows) {
@@ -531,10 +634,10 @@ static int run_group_qmv(const Group& g, const void* x, int x_type, int64_t rows
   return check_launch("EXL3 QMV launch");
 }
 
-// Prologue (one launch for all members) and one QMM launch over the group.
+// Prologue (one launch for all members) and one QMM over the group.
 // xhats: per member, null to run the prologue into the scratch.
 static int run_group_qmm(const Group& g, const void* x, int x_type, int64_t rows,
-                         void* const* ys, uint32_t* counters, char* scratch,
+                         void* const* ys, uint32_t* counters, char* scratch, size_t scratch_bytes,
                          const uint16_t* given_xhat, hipStream_t stream) {
   if (int rc = launch_gate("EXL3 QMM launch")) return rc;
   const size_t xbytes = align_up(sizeof(uint16_t) * (size_t)rows * g.in);
@@ -558,9 +661,35 @@ static int run_group_qmm(const Group& g, const void* x, int x_type, int64_t rows
     q.mem[i].xhat = given_xhat ? given_xhat : (const uint16_t*)(scratch + i * xbytes);
     cblk0 += g.parts[i]->out / 128;
   }
+  const size_t xhats = given_xhat ? 0 : g.count * xbytes;
+  WideShape ws;
+  if (group_takes_wide(g, rows, std::min(group_partial_budget(g, rows), scratch_bytes - xhats),
+                       &ws) && ((uintptr_t)q.mem[0].xhat & 15) == 0) {
+    WideParams w{};
+    for (int i = 0; i < g.count; ++i) {
+      const Member& m = q.mem[i];
+      w.mem[i] = WideMember{m.trellis, m.xhat, m.svh, m.bias, m.y, m.out, w.pairs, m.y_dtype};
+      w.pairs += (m.out + 255) / 256;
+    }
+    w.members = g.count;
+    w.partials = (float*)(scratch + xhats);
+    w.in = g.in;
+    w.M = (int)rows;
+    w.x_dtype = x_type;
+    w.mtiles = ws.mtiles;
+    w.splits = ws.splits;
+    const int64_t wgs = (int64_t)w.mtiles * w.pairs * w.splits;
+    if (wgs > INT32_MAX) return fail(EXL3_EINVAL, "EXL3 QMM grid too large");
+    kWide[ws.r == 16 ? 2 : ws.r == 8 ? 1 : 0][g.k - 1][g.cb](w, dim3((unsigned)wgs), stream);
+    if (w.splits > 1) {
+      if (int rc = check_launch("EXL3 QMM launch")) return rc;
+      launch_wide_reduce(w, ws.r, stream);
+    }
+    return check_launch("EXL3 QMM launch");
+  }
   const QmmShape sh = choose_qmm_shape(g.in, g.total_out, rows);
   q.members = g.count;
-  q.partials = (float*)(scratch + (given_xhat ? 0 : g.count * xbytes));
+  q.partials = (float*)(scratch + xhats);
   q.counters = counters;
   q.in = g.in;
   q.total_out = g.total_out;
@@ -583,14 +712,15 @@ static int group_forward(const Group& g, const void* x, int x_type, int64_t rows
     if (!ys[i]) return fail(EXL3_EINVAL, "null activation pointer");
   if (!valid_dtype(x_type)) return fail(EXL3_EINVAL, "unsupported activation dtype code %d", x_type);
   if (int rc = check_rows(g, rows)) return rc;
-  const size_t need = kWorkspaceCounterBytes + group_scratch_bytes(g, rows);
+  const size_t need = kWorkspaceCounterBytes + group_scratch_min(g, rows);
   if (!ws || ws_bytes < need)
     return fail(EXL3_EINVAL, "workspace too small: %zu bytes given, %zu needed", ws_bytes, need);
   uint32_t* counters = (uint32_t*)ws;
   char* scratch = (char*)ws + kWorkspaceCounterBytes;
   const Glu none{};
   if (rows <= kQmvMaxRows) return run_group_qmv(g, x, x_type, rows, ys, counters, scratch, none, stream);
-  return run_group_qmm(g, x, x_type, rows, ys, counters, scratch, nullptr, stream);
+  return run_group_qmm(g, x, x_type, rows, ys, counters, scratch,
+                       ws_bytes - kWorkspaceCounterBytes, nullptr, stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -612,22 +742,20 @@ static int mlp_check(const exl3_linear* gate, const exl3_linear* up, const exl3_
   return EXL3_OK;
 }
 
+// `least`: what a call cannot do without, else what it makes use of.
 static size_t mlp_ws_bytes(const exl3_linear* gate, const exl3_linear* up,
-                           const exl3_linear* down, int64_t rows) {
+                           const exl3_linear* down, int64_t rows, bool least) {
   const exl3_linear* gu[2] = {gate, up};
-  Group g;
-  if (make_group(gu, 2, g)) return 0;
+  Group g, d;
+  if (make_group(gu, 2, g) || make_group(&down, 1, d)) return 0;
   const size_t act = align_up(sizeof(uint16_t) * (size_t)rows * gate->out);
   size_t need;
   if (rows <= kQmvMaxRows) {
-    Group d;
-    if (make_group(&down, 1, d)) return 0;
     need = act + std::max(group_scratch_bytes(g, rows), group_scratch_bytes(d, rows));
   } else {
-    const QmmShape sh = choose_qmm_shape(down->in, down->out, rows);
-    const size_t stage2 = align_up(qmm_partial_bytes(sh, down->out));
     // down xhat + gate and up outputs
-    need = 3 * act + std::max(group_scratch_bytes(g, rows), stage2);
+    need = 3 * act + (least ? std::max(group_scratch_min(g, rows), align_up(group_qmm_partials_min(d, rows)))
+                            : std::max(group_scratch_bytes(g, rows), align_up(group_qmm_partials(d, rows))));
   }
   return kWorkspaceCounterBytes + need;
 }
@@ -646,7 +774,7 @@ static int mlp_forward(const exl3_linear* gate, const exl3_linear* up, const exl
   if (int rc = make_group(&down, 1, d)) return rc;
   if (int rc = check_rows(g, rows)) return rc;
   if (int rc = check_rows(d, rows)) return rc;
-  const size_t need = mlp_ws_bytes(gate, up, down, rows);
+  const size_t need = mlp_ws_bytes(gate, up, down, rows, true);
   if (!ws || ws_bytes < need)
     return fail(EXL3_EINVAL, "workspace too small: %zu bytes given, %zu needed", ws_bytes, need);
   uint32_t* counters = (uint32_t*)ws;
@@ -674,13 +802,16 @@ static int mlp_forward(const exl3_linear* gate, const exl3_linear* up, const exl
   }
   void* gu_y[2] = {base + act_bytes, base + 2 * act_bytes};
   char* scratch = base + 3 * act_bytes;
-  if (int rc = run_group_qmm(g, x, EXL3_F16, rows, gu_y, counters, scratch, nullptr, stream))
+  const size_t scratch_bytes = ws_bytes - kWorkspaceCounterBytes - 3 * act_bytes;
+  if (int rc = run_group_qmm(g, x, EXL3_F16, rows, gu_y, counters, scratch, scratch_bytes, nullptr,
+                             stream))
     return rc;
   if (int rc = launch_gate("SwiGLU prepare launch")) return rc;
   launch_swiglu_prepare((const uint16_t*)gu_y[0], (const uint16_t*)gu_y[1], down->suh, gate->out,
                         (int)rows, act, stream);
   if (int rc = check_launch("SwiGLU prepare launch")) return rc;
-  return run_group_qmm(d, nullptr, EXL3_F16, rows, dy, counters, scratch, act, stream);
+  return run_group_qmm(d, nullptr, EXL3_F16, rows, dy, counters, scratch, scratch_bytes, act,
+                       stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -747,7 +878,7 @@ size_t exl3_group_workspace_bytes(const exl3_linear* const* parts, int32_t count
 size_t exl3_mlp_workspace_bytes(const exl3_linear* gate, const exl3_linear* up,
                                 const exl3_linear* down, int64_t rows) {
   if (rows < 1 || mlp_check(gate, up, down)) return 0;
-  return mlp_ws_bytes(gate, up, down, rows);
+  return mlp_ws_bytes(gate, up, down, rows, false);
 }
 
 int exl3_workspace_init(void* workspace, size_t bytes, void* stream) {
@@ -787,7 +918,7 @@ int exl3_linear_forward_noalloc(const exl3_linear* h, const void* x, int32_t x_t
   Group g;
   if (int rc = make_group(&h, 1, g)) return rc;
   if (int rc = check_rows(g, rows)) return rc;
-  const size_t need = kWorkspaceCounterBytes + group_scratch_bytes(g, rows);
+  const size_t need = kWorkspaceCounterBytes + group_scratch_min(g, rows);
   if (need > kNoAllocBytes)
     return fail(EXL3_EUNSUPPORTED,
                 "allocation-free EXL3 forward of %lld rows needs %zu bytes of workspace, more "

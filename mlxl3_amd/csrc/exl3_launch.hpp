@@ -15,6 +15,7 @@ namespace exl3 {
 
 typedef void (*QmvFn)(const QmvParams&, dim3, size_t, hipStream_t);
 typedef void (*QmmFn)(const QmmParams&, dim3, hipStream_t);
+typedef void (*WideFn)(const WideParams&, dim3, hipStream_t);
 typedef void (*DecodeFn)(const uint32_t*, int64_t, uint16_t*, uint16_t*, dim3, hipStream_t);
 
 // Every workspace starts with this many bytes of counters that are zero
@@ -32,8 +33,13 @@ extern const QmvFn kQmvFragShallow[8][3];  // kQmvFrag with one slice per prefet
 extern const DecodeFn kDecode[8][3];
 extern const QmmFn kQmm[3][8][3];  // [log2 MB]: 64, 128 or 256 rows per workgroup
 
+extern const WideFn kWide[3][8][3];  // [log2(R / 4)]: 64, 128 or 256 rows per workgroup
+
 // xhat of `members` (suh, xhat) pairs of p in one launch.
 void launch_prologue(const PrologueParams& p, int members, hipStream_t s);
+// Sums the split-K partials of a kWide launch of 16*R rows per workgroup and
+// finishes its outputs.
+void launch_wide_reduce(const WideParams& p, int R, hipStream_t s);
 // values[i] = codeword(states[i], cb).
 void launch_codewords(const uint16_t* states, int64_t n, int cb, uint16_t* values, hipStream_t s);
 // packed[t][16k] = the trellis tile of states[t][256] (low k bits of each).

@@ -57,6 +57,27 @@ struct QmmParams {
   int splits;          // K-ranges per output tile (global split-K)
 };
 
+// A projection of a wide QMM launch: it owns the column pairs (256 columns)
+// [pair0, pair0 + ceil(out / 256)).
+struct WideMember {
+  const uint32_t* trellis;
+  const uint16_t* xhat;  // [M][in] f16
+  const uint16_t* svh;
+  const uint16_t* bias;
+  void* y;
+  int out, pair0, y_dtype;
+};
+struct WideParams {
+  WideMember mem[kMaxMembers];
+  int members;
+  float* partials;     // [splits][tiles][16*R x 256 f32 in fragment order] (splits > 1)
+  uint32_t* counters;  // [mtiles * pairs], zero between calls (splits > 1)
+  int in, M, x_dtype;
+  int pairs;   // column pairs of all members
+  int mtiles;  // ceil(M / rows per workgroup)
+  int splits;
+};
+
 struct PrologueParams {
   const void* x;  // [rows][in] of x_dtype
   int x_dtype, in, rows;
@@ -74,6 +95,15 @@ __device__ __forceinline__ Member select_member(const P& p, int cblk) {
 #pragma unroll
   for (int i = 1; i < kMaxMembers; ++i)
     if (i < p.members && cblk >= p.mem[i].cblk0) m = p.mem[i];
+  return m;
+}
+
+template <typename P>
+__device__ __forceinline__ WideMember select_wide(const P& p, int pair) {
+  WideMember m = p.mem[0];
+#pragma unroll
+  for (int i = 1; i < kMaxMembers; ++i)
+    if (i < p.members && pair >= p.mem[i].pair0) m = p.mem[i];
   return m;
 }
 

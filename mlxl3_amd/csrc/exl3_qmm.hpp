@@ -20,7 +20,7 @@
 //
 // After the loop the consumers round their accumulators to f16 rows in LDS and
 // all 8 waves run the output epilogue (f16 -> staged H128 -> * svh -> cast,
-// linear.rs:1940-1963) with 8 consecutive columns per lane.  With a global
+// linear.rs:1940-1963; qmm_finish16).  With a global
 // split-K the K-ranges leave f32 partials (exchanged with agent-scope relaxed
 // atomics, as in the QMV) and the last workgroup of an output tile adds them
 // in split order, so results do not depend on timing.
@@ -112,27 +112,27 @@ __global__ __launch_bounds__(256) void swiglu_prepare_kernel(const uint16_t* __r
 }
 
 // Rows of a finished tile pass through LDS as f16: Y[row][136] (128 columns
-// plus 8 halves of padding, so the 16-byte reads of one row never meet the
-// next row's banks).
+// plus 8 halves of padding: the 8-byte reads of 16 rows then touch every bank
+// once).  The columns of a 16-column tile sit at position 2*(c % 8) + c / 8, which
+// puts the two values that a lane holds of a row (columns c and c + 8) into one
+// dword.
 constexpr int kYStride = 136;
 
+typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+typedef float float2v __attribute__((ext_vector_type(2)));
+
+// Two f32 values rounded to f16 (one instruction), and such a pair as f32.
+__device__ __forceinline__ half2v pack_f16(float a, float b) {
+  return __builtin_convertvector(float2v{a, b}, half2v);
+}
+
 // Consumer side: f16(acc) of one row into Y.  Register f of the lane holds
-// column 32*(f>>1) + 8*(f&1) + lanecol, lanecol = 16*(n>>3) + (n&7), n =
-// lane & 15.  Neighbouring lanes swap one value so that each lane writes two
-// 32-bit column pairs: an even lane columns (c, c+1) of register 2w, an odd
-// lane columns (c-1, c) of register 2w+1.
+// column 32*(f>>1) + 8*(f&1) + 16*(n>>3) + (n&7), n = lane & 15.
 __device__ __forceinline__ void qmm_stage_row(const float (&v)[8], int lane, uint16_t* yrow) {
   const int n = lane & 15;
-  const bool odd = n & 1;
-  const int pcol = 16 * (n >> 3) + (n & 7) + (odd ? 7 : 0);
-  uint32_t* y32 = (uint32_t*)(yrow + pcol);
+  uint16_t* y = yrow + 16 * (n >> 3) + 2 * (n & 7);
 #pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    const float mine = odd ? v[2 * w + 1] : v[2 * w];
-    const float other = xor_lanes<1>(odd ? v[2 * w] : v[2 * w + 1]);
-    const float lo = odd ? other : mine, hi = odd ? mine : other;
-    y32[16 * w] = (uint32_t)f2h(lo) | ((uint32_t)f2h(hi) << 16);
-  }
+  for (int w = 0; w < 4; ++w) *(half2v*)(y + 32 * w) = pack_f16(v[2 * w], v[2 * w + 1]);
 }
 
 // Value of the linear epilogue's final cast (+ bias), as out_value computes
@@ -148,44 +148,99 @@ __device__ __forceinline__ uint32_t out16(float v, int y_dt) {
   return y_dt == DT_F16 ? f2h(v) : f2bf(v);
 }
 
-// Finishing side: each lane holds 8 consecutive columns 8*(lane&15)+j of one
-// row (four rows per wave pass): f16 values -> staged Hadamard-128 (strides
-// 1, 2, 4 inside the lane, 8..64 across lanes 1..8, f16 rounding after
-// strides 8 and 64) -> f16(* 1/sqrt 128) -> f16(* svh) -> cast (+ bias) ->
-// one 16-byte store (two for f32).  sv/bv: svh and bias of the lane's columns.
-__device__ __forceinline__ void qmm_finish_chunk(const u32x4 raw, const float (&sv)[8],
-                                                 const float (&bv)[8], int lane, bool live,
-                                                 const Member& mm, int x_dtype, size_t yoff) {
-  float v[8];
+// Where a projection's output goes and how it is cast.
+struct QmmOut {
+  void* y;
+  int y_dtype;
+  bool has_bias;
+};
+
+// Output epilogue of 16 staged rows x 128 columns (first row, first column at
+// `ys`): f16 -> staged H128 -> f16(* 1/sqrt 128) -> f16(* svh) -> cast (+ bias)
+// -> y (linear.rs:984-997, :1940-1963).  Strides 1..8 of the Hadamard are one
+// MFMA per 16 columns (H16 x the transposed rows: sums of 16 f16 values in f32),
+// strides 16..64 adds between the 8 results of a lane, with f16 rounding after
+// each half as the staged transform has it.  Lane (g, n) ends with columns 16i +
+// 4g + 0..3 of row n.  ~9 VALU instructions per value, where the transform by
+// lane exchanges takes ~30.
+// RN = 2: only columns 4g + r0, r0 + 1 of each 4 (two waves share the rows).
+template <int RN = 4>
+__device__ __forceinline__ void qmm_finish16(const uint16_t* ys, int stride, const uint16_t* svh,
+                                             const uint16_t* bias, int lane, bool live,
+                                             const QmmOut& out, int x_dtype, size_t yoff,
+                                             int r0 = 0) {
+  const int g = lane >> 4, n = lane & 15;
+  half4 hm;  // H16 row n at the true columns of positions 4g + i
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    v[2 * i] = h2f((uint16_t)raw[i]);
-    v[2 * i + 1] = h2f((uint16_t)(raw[i] >> 16));
+    const int c = 2 * g + (i >> 1) + 8 * (i & 1);
+    hm[i] = (__builtin_popcount(c & n) & 1) ? -1.f : 1.f;
   }
-  h128_lane8(v, lane);
+  float v[8][RN];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) v[j] = round_f16(round_f16(v[j] * kHadScale) * sv[j]);
-  if (!live) return;
-  const bool has_bias = mm.bias != nullptr;
+  for (int i = 0; i < 8; ++i) {
+    const half4 yr = *(const half4*)(ys + n * stride + 16 * i + 4 * g);
+    float4v d =
+        __builtin_amdgcn_mfma_f32_16x16x16f16(hm, yr, float4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+    if (RN == 2 && r0) d[0] = d[2], d[1] = d[3];  // uniform
 #pragma unroll
-  for (int j = 0; j < 8; ++j) v[j] = out_cast(v[j], bv[j], has_bias, x_dtype);
-  if (mm.y_dtype == DT_F32) {
-    float4v o0, o1;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      o0[j] = v[j];
-      o1[j] = v[j + 4];
+    for (int r = 0; r < RN; r += 2) {
+      const half2v h = pack_f16(d[r], d[r + 1]);
+      v[i][r] = (float)h[0];
+      v[i][r + 1] = (float)h[1];
     }
-    float4v* yp = (float4v*)((float*)mm.y + yoff);
-    yp[0] = o0;
-    yp[1] = o1;
-    return;
   }
-  u32x4 o;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-    o[i] = out16(v[2 * i], mm.y_dtype) | (out16(v[2 * i + 1], mm.y_dtype) << 16);
-  *(u32x4*)((uint16_t*)mm.y + yoff) = o;
+  for (int s = 1; s < 8; s <<= 1)
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (!(i & s))
+#pragma unroll
+        for (int r = 0; r < RN; ++r) {
+          const float p = v[i][r], q = v[i + s][r];
+          v[i][r] = p + q;
+          v[i + s][r] = p - q;
+        }
+  const bool plain = !out.has_bias && x_dtype == DT_F16;  // uniform
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int c = 16 * i + 4 * g + r0;
+    half2v o[RN / 2];
+#pragma unroll
+    for (int r = 0; r < RN / 2; ++r) {
+      const half2v h = pack_f16(v[i][2 * r], v[i][2 * r + 1]);
+      // the f32 product of two f16 values is exact: its rounding is the f16 product
+      o[r] = pack_f16((float)h[0] * kHadScale, (float)h[1] * kHadScale) *
+             *(const half2v*)(svh + c + 2 * r);
+    }
+    if (!live) continue;
+    uint32_t w[RN / 2];
+    if (plain) {
+#pragma unroll
+      for (int r = 0; r < RN / 2; ++r) w[r] = __builtin_bit_cast(uint32_t, o[r]);
+    } else {
+      float f[RN];
+#pragma unroll
+      for (int r = 0; r < RN; ++r)
+        f[r] = out_cast((float)o[r >> 1][r & 1], h2f(bias[c + r]), out.has_bias, x_dtype);
+      if (out.y_dtype == DT_F32) {
+        float* y = (float*)out.y + yoff + c;
+        if constexpr (RN == 4)
+          *(float4v*)y = float4v{f[0], f[1], f[2], f[3]};
+        else
+          *(float2v*)y = float2v{f[0], f[1]};
+        continue;
+      }
+#pragma unroll
+      for (int r = 0; r < RN / 2; ++r)
+        w[r] = out16(f[2 * r], out.y_dtype) | (out16(f[2 * r + 1], out.y_dtype) << 16);
+    }
+    uint16_t* y = (uint16_t*)out.y + yoff + c;
+    if constexpr (RN == 4)
+      *(u32x2*)y = u32x2{w[0], w[1]};
+    else
+      *(uint32_t*)y = w[0];
+  }
 }
 
 // load_slice_prev<K> as raw buffer loads with a fixed count of load
@@ -257,7 +312,7 @@ __global__ __launch_bounds__(512) void qmm_kernel(QmmParams p) {
   __shared__ __attribute__((aligned(16))) uint8_t bls[3 * kBStage];
   __shared__ __attribute__((aligned(16))) uint8_t als[kABytes];
   uint16_t* ys = (uint16_t*)als;  // [64*MB][kYStride] after the loop
-  __shared__ float s_svh[128], s_bias[128];
+  __shared__ __attribute__((aligned(16))) uint16_t s_svh[128], s_bias[128];
   __shared__ int s_last;
   auto bstage = [&](int st) { return (u32x4*)(bls + st * kBStage); };  // [producer][frag][lane]
   auto astage = [&](int st) { return als + st * kAStage; };
@@ -301,8 +356,8 @@ __global__ __launch_bounds__(512) void qmm_kernel(QmmParams p) {
     // ---- producer `role`: B tiles of output tiles 2*role, 2*role+1 and the
     // A rows of consumer `role` ----
     if (threadIdx.x < 128) {
-      s_svh[threadIdx.x] = h2f(mm.svh[cblk_l * 128 + threadIdx.x]);
-      s_bias[threadIdx.x] = mm.bias ? h2f(mm.bias[cblk_l * 128 + threadIdx.x]) : 0.f;
+      s_svh[threadIdx.x] = mm.svh[cblk_l * 128 + threadIdx.x];
+      s_bias[threadIdx.x] = mm.bias ? mm.bias[cblk_l * 128 + threadIdx.x] : 0;
     }
     // trellis slices in flight: 4 steps ahead (with A copied straight to LDS
     // at MB >= 2 no variant spills at this depth)
@@ -532,7 +587,7 @@ __global__ __launch_bounds__(512) void qmm_kernel(QmmParams p) {
         for (int r = 0; r < 4; ++r) {
           float v[8];
 #pragma unroll
-          for (int f = 0; f < 8; ++f) v[f] = round_f16(acc[mb][f][r]);
+          for (int f = 0; f < 8; ++f) v[f] = acc[mb][f][r];
           qmm_stage_row(v, lane, ys + (role * 16 * MB + 16 * mb + 4 * g + r) * kYStride);
         }
       });
@@ -563,7 +618,7 @@ __global__ __launch_bounds__(512) void qmm_kernel(QmmParams p) {
     // round trip to the coherence point per group, not per load), its four
     // rows rounded to f16 into the tile's rows in LDS
     constexpr int kSumFrags = 4, kSumParts = 4;
-    const int col = 16 * (n >> 3) + (n & 7);
+    const int col = 16 * (n >> 3) + 2 * (n & 7);
     for (int i0 = 0; i0 < 4 * MB; i0 += kSumFrags) {
       float4v sum[kSumFrags];
 #pragma unroll
@@ -590,7 +645,7 @@ __global__ __launch_bounds__(512) void qmm_kernel(QmmParams p) {
         const int slot = wave * 4 * MB + i0 + i;  // (consumer, mb, f)
         const int cr = slot / (8 * MB), mb = (slot / 8) % MB, f = slot % 8;
         uint16_t* y = ys + (cr * 16 * MB + 16 * mb + 4 * g) * kYStride + 32 * (f >> 1) +
-                      8 * (f & 1) + col;
+                      (f & 1) + col;
 #pragma unroll
         for (int r = 0; r < 4; ++r) y[r * kYStride] = f2h(sum[i][r]);
       }
@@ -598,24 +653,15 @@ __global__ __launch_bounds__(512) void qmm_kernel(QmmParams p) {
   }
   __syncthreads();
 
-  // ---- epilogue: all 8 waves finish 8*MB rows each, 4 rows per pass ----
-  {
-    const int colb = cblk_l * 128;
-    const int chunk = lane & 15;
-    float sv[8], bv[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      sv[j] = s_svh[8 * chunk + j];
-      bv[j] = s_bias[8 * chunk + j];
-    }
-#pragma unroll
-    for (int i = 0; i < 2 * MB; ++i) {
-      const int rl = wave * 8 * MB + 4 * i + (lane >> 4);
-      const int row = mtile * 64 * MB + rl;
-      const u32x4 raw = *(const u32x4*)(ys + rl * kYStride + 8 * chunk);
-      qmm_finish_chunk(raw, sv, bv, lane, row < p.M, mm, p.x_dtype,
-                       (size_t)row * mm.out + colb + 8 * chunk);
-    }
+  // ---- epilogue: 4*MB row groups of 16 over the 8 waves (MB = 1: two waves
+  // each, sharing the columns) ----
+  const QmmOut out{mm.y, mm.y_dtype, mm.bias != nullptr};
+  constexpr int kShare = MB == 1 ? 2 : 1;
+  for (int u = wave / kShare; u < 4 * MB; u += 8 / kShare) {
+    const int row = mtile * 64 * MB + 16 * u + n;
+    qmm_finish16<4 / kShare>(ys + 16 * u * kYStride, kYStride, s_svh, s_bias, lane, row < p.M, out,
+                             p.x_dtype, (size_t)row * mm.out + cblk_l * 128,
+                             kShare == 2 ? 2 * (wave & 1) : 0);
   }
 }
 
