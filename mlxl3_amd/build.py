@@ -23,7 +23,8 @@ HERE = Path(__file__).resolve().parent
 CSRC = HERE / "csrc"
 LIB = HERE / "libexl3_hip.so"
 CODEC = HERE / "exl3_codec"  # the codec JSON-lines driver (links LIB)
-SOURCES = ["exl3_api.hip", "exl3_qmv.hip", "exl3_qmm.hip", "exl3_wide.hip", "exl3_moe.hip", "exl3_mapped.hip",
+SOURCES = ["exl3_api.hip", "exl3_qmv.hip", "exl3_qmm.hip", "exl3_wide.hip", "exl3_moe.hip", "exl3_moe_wide.hip",
+           "exl3_mapped.hip",
            "exl3_checkpoint.cpp"]
 ARCH = "gfx950"
 

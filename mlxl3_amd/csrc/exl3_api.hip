@@ -318,51 +318,61 @@ static size_t qmm_partial_bytes(const QmmShape& sh, int out) {
   return sizeof(float) * (size_t)sh.splits * sh.mtiles * (out / 128) * 64 * sh.mb * 128;
 }
 
-// Launch shape of the decode-in-registers QMM (exl3_wide.hpp): 16*R rows x 256
-// columns per workgroup, one workgroup per CU at R = 8 and 16, two at R = 4.
-// Rounds of workgroups x (steps of 64 inputs per split) x the step time (ns,
-// every CU busy: R = 4 1500 with two workgroups, 8 1060, 16 1560), a fixed part
-// per launch (ring fill, epilogue, output flush: 8 / 9 / 15 us) and, with
-// splits, 3 us and 0.42 ns per KB of f32 partials for the summing launch.
-// Measured against the producer/consumer kernel on one box (us, the better shape
-// of each): 4096x28672 M 384/512/1024/2048 162/159/322/578 -> 120/126/246/494,
-// 14336x4096 M 256/512/1024/4096 61/98/160/567 -> 55/87/147/482, 27648x5120 M
-// 256/512/2048 116/196/939 -> 103/169/602, 5120x7168 M 384/2048 67/202 ->
-// 53/159; it loses on small launches (2048x1536 M 64..1024 16-32 -> 18-33,
-// 4096x4096 M 64/128 21/24 -> 24/28), where its 256-column tiles are too few.
+// Launch shape of the decode-in-registers QMM (exl3_wide.hpp): tiles of 64 rows x
+// 128 columns (two workgroups per CU), 128 x 256 or 256 x 256 (one).  Rounds of
+// workgroups x steps of 64 inputs per split x the step time, a fixed part per
+// launch and, with splits, 3 us and 0.42 ns per KB of f32 partials for the summing
+// launch; fitted to a sweep of every tile and split count over seven shapes x 32 to
+// 4096 rows at K = 4 (one box), where it is within 3 % of the fastest measured but
+// where the partials of more splits would pass the allocation-free entry point's
+// budget.  Against the producer/consumer kernel there (us, calls): 4096x28672 rows
+// 384/512/1024/2048 147/142/285/521 -> 112/117/228/461, 14336x4096 rows
+// 768/2048/4096 126/259/524 -> 111/247/442, 27648x5120 rows 384/512/1024
+// 167/175/339 -> 138/158/287, 5120x7168 rows 2048/4096 185/353 -> 148/289, 4096x14336
+// rows 64/768/2048 32.3/146/285 -> 29.7/105/230; that kernel keeps most launches of
+// few tiles (2048x1536 rows 256..2048 19.3-37.1 against 20.4-37.4, 4096x4096 rows 256
+// 29.3 against 30.7), where 256-column tiles leave CUs idle.
 struct WideShape {
-  int r, mtiles, splits;
+  int kind, mtiles, splits;  // kind: index of kWide and kWideTiles
   double cost;
 };
+struct WideTile {
+  int r, nw, per_cu;          // 16*r rows x 32*nw columns, workgroups per CU
+  double step_ns, alone_ns;   // a step with every CU full, and with one workgroup each
+  double fixed_ns;            // ring fill, epilogue and output flush of a launch
+};
+static constexpr WideTile kWideTiles[3] = {{4, 4, 2, 1000, 750, 5000},
+                                           {8, 8, 1, 1060, 1060, 9000},
+                                           {16, 8, 1, 1560, 1560, 15000}};
 
-static size_t wide_partial_bytes(int r, int mtiles, int pairs, int splits) {
-  return splits > 1 ? sizeof(float) * (size_t)splits * mtiles * pairs * 16 * r * 256 : 0;
+static size_t wide_partial_bytes(const WideTile& t, int64_t mtiles, int units, int splits) {
+  return splits > 1 ? sizeof(float) * (size_t)splits * mtiles * units * 16 * t.r * 32 * t.nw : 0;
 }
 
-// The cheapest shape whose partials fit in `budget` bytes (one split always fits).
-static WideShape choose_wide_shape(int in, int pairs, int64_t rows, size_t budget) {
+// The cheapest shape whose partials fit in `budget` bytes (one split always fits);
+// units[i]: column units of the launch in tiles of 128 (0) or 256 (1) columns.
+static WideShape choose_wide_shape(int in, const int (&units)[2], int64_t rows, size_t budget) {
   const int nq = in / 64;
-  int force_r = 0, force_splits = 0;
-  if (const char* env = getenv("EXL3_WIDE_R")) force_r = atoi(env);
+  int force_kind = -1, force_splits = 0;
+  if (const char* env = getenv("EXL3_WIDE_TILE")) force_kind = std::max(0, std::min(atoi(env), 2));
   if (const char* env = getenv("EXL3_WIDE_SPLITS")) force_splits = std::max(0, atoi(env));
-  WideShape best{16, (int)((rows + 255) / 256), 1, 1e300};
-  for (int r : {4, 8, 16}) {
-    if (force_r && r != force_r) continue;
-    const int64_t mt = (rows + 16 * r - 1) / (16 * r);
-    const int per_round = r == 4 ? 512 : 256;
-    const double step_ns = r == 4 ? 1500.0 : r == 8 ? 1060.0 : 1560.0;
-    const double fixed = r == 4 ? 8000.0 : r == 8 ? 9000.0 : 15000.0;
+  WideShape best{2, (int)((rows + 255) / 256), 1, 1e300};
+  for (int kind = 0; kind < 3; ++kind) {
+    if (force_kind >= 0 && kind != force_kind) continue;
+    const WideTile& t = kWideTiles[kind];
+    const int u = units[t.nw / 8];
+    const int64_t mt = (rows + 16 * t.r - 1) / (16 * t.r);
     for (int splits = 1; splits <= 8; ++splits) {
       int sp = force_splits ? force_splits : splits;
       sp = std::max(1, std::min(sp, std::max(1, nq / 4)));
-      const size_t part = wide_partial_bytes(r, (int)mt, pairs, sp);
+      const size_t part = wide_partial_bytes(t, mt, u, sp);
       if (part > budget) continue;
-      const int64_t wgs = mt * pairs * sp, rounds = (wgs + per_round - 1) / per_round;
-      // half-empty CUs of an R = 4 launch run their one workgroup faster
-      const double step = r == 4 && wgs <= 256 ? 900.0 : step_ns;
-      double cost = fixed + (double)rounds * ((nq + sp - 1) / sp) * step;
+      const int64_t wgs = mt * u * sp;
+      const int64_t rounds = (wgs + 256 * t.per_cu - 1) / (256 * t.per_cu);
+      const double step = wgs <= 256 ? t.alone_ns : t.step_ns;
+      double cost = t.fixed_ns + (double)rounds * ((nq + sp - 1) / sp) * step;
       if (sp > 1) cost += 3000.0 + 0.42 / 1024 * (double)part;
-      if (cost < best.cost) best = WideShape{r, (int)mt, sp, cost};
+      if (cost < best.cost) best = WideShape{kind, (int)mt, sp, cost};
       if (force_splits) break;
     }
   }
@@ -447,11 +457,12 @@ static bool qmv_fragment_exchange(int64_t rows, int kw) {
   return kw == 1 && rows >= from;
 }
 
-// Column pairs (256 columns) of a group: a member's last one may be half empty.
-static int group_pairs(const Group& g) {
-  int pairs = 0;
-  for (int i = 0; i < g.count; ++i) pairs += (g.parts[i]->out + 255) / 256;
-  return pairs;
+// Column units of a group in tiles of `cols` columns (a member's last one may be
+// half empty).
+static int group_units(const Group& g, int cols) {
+  int units = 0;
+  for (int i = 0; i < g.count; ++i) units += (g.parts[i]->out + cols - 1) / cols;
+  return units;
 }
 
 // Whether a QMM over the group runs in registers (exl3_wide.hpp) and in which
@@ -463,7 +474,8 @@ static int group_pairs(const Group& g) {
 static bool group_takes_wide(const Group& g, int64_t rows, size_t budget, WideShape* shape) {
   for (int i = 0; i < g.count; ++i)
     if ((uintptr_t)g.parts[i]->trellis & 15) return false;
-  *shape = choose_wide_shape(g.in, group_pairs(g), rows, budget);
+  const int units[2] = {group_units(g, 128), group_units(g, 256)};
+  *shape = choose_wide_shape(g.in, units, rows, budget);
   if (const char* env = getenv("EXL3_WIDE")) return atoi(env) != 0;
   return shape->cost < choose_qmm_shape(g.in, g.total_out, rows).cost + 6000.0;
 }
@@ -489,7 +501,8 @@ static size_t group_qmm_partials(const Group& g, int64_t rows) {
   WideShape sh;
   const size_t least = group_qmm_partials_min(g, rows);
   if (!group_takes_wide(g, rows, group_partial_budget(g, rows), &sh)) return least;
-  return std::max(least, wide_partial_bytes(sh.r, sh.mtiles, group_pairs(g), sh.splits));
+  const WideTile& t = kWideTiles[sh.kind];
+  return std::max(least, wide_partial_bytes(t, sh.mtiles, group_units(g, 32 * t.nw), sh.splits));
 }
 
 // Scratch bytes (after the counter region) of one group launch.
@@ -652,7 +665,7 @@ static int run_group_qmm(const Group& g, const void* x, int x_type, int64_t rows
       pp.suh[i] = g.parts[i]->suh;
       pp.xhat[i] = (uint16_t*)(scratch + i * xbytes);
     }
-    launch_prologue(pp, g.count, stream);
+    launch_prologue16(pp, g.count, stream);
     if (int rc = check_launch("EXL3 prologue launch")) return rc;
   }
   int cblk0 = 0;
@@ -665,11 +678,12 @@ static int run_group_qmm(const Group& g, const void* x, int x_type, int64_t rows
   WideShape ws;
   if (group_takes_wide(g, rows, std::min(group_partial_budget(g, rows), scratch_bytes - xhats),
                        &ws) && ((uintptr_t)q.mem[0].xhat & 15) == 0) {
+    const WideTile& t = kWideTiles[ws.kind];
     WideParams w{};
     for (int i = 0; i < g.count; ++i) {
       const Member& m = q.mem[i];
-      w.mem[i] = WideMember{m.trellis, m.xhat, m.svh, m.bias, m.y, m.out, w.pairs, m.y_dtype};
-      w.pairs += (m.out + 255) / 256;
+      w.mem[i] = WideMember{m.trellis, m.xhat, m.svh, m.bias, m.y, m.out, w.units, m.y_dtype};
+      w.units += (m.out + 32 * t.nw - 1) / (32 * t.nw);
     }
     w.members = g.count;
     w.partials = (float*)(scratch + xhats);
@@ -678,12 +692,12 @@ static int run_group_qmm(const Group& g, const void* x, int x_type, int64_t rows
     w.x_dtype = x_type;
     w.mtiles = ws.mtiles;
     w.splits = ws.splits;
-    const int64_t wgs = (int64_t)w.mtiles * w.pairs * w.splits;
+    const int64_t wgs = (int64_t)w.mtiles * w.units * w.splits;
     if (wgs > INT32_MAX) return fail(EXL3_EINVAL, "EXL3 QMM grid too large");
-    kWide[ws.r == 16 ? 2 : ws.r == 8 ? 1 : 0][g.k - 1][g.cb](w, dim3((unsigned)wgs), stream);
+    kWide[ws.kind][g.k - 1][g.cb](w, dim3((unsigned)wgs), stream);
     if (w.splits > 1) {
       if (int rc = check_launch("EXL3 QMM launch")) return rc;
-      launch_wide_reduce(w, ws.r, stream);
+      launch_wide_reduce(w, t.r, t.nw, stream);
     }
     return check_launch("EXL3 QMM launch");
   }

@@ -16,6 +16,12 @@ namespace exl3 {
 typedef void (*QmvFn)(const QmvParams&, dim3, size_t, hipStream_t);
 typedef void (*QmmFn)(const QmmParams&, dim3, hipStream_t);
 typedef void (*WideFn)(const WideParams&, dim3, hipStream_t);
+struct MoeMmParams;
+struct MoePlanParams;
+struct MoeGatherParams;
+// (parameters, gate/up with the GLU edge or down, blocks rounded up to 8, the
+// edge's [2][slots][hidden] f16 scratch, stream)
+typedef void (*MoeWideFn)(const MoeMmParams&, bool, int, uint16_t*, hipStream_t);
 typedef void (*DecodeFn)(const uint32_t*, int64_t, uint16_t*, uint16_t*, dim3, hipStream_t);
 
 // Every workspace starts with this many bytes of counters that are zero
@@ -33,13 +39,20 @@ extern const QmvFn kQmvFragShallow[8][3];  // kQmvFrag with one slice per prefet
 extern const DecodeFn kDecode[8][3];
 extern const QmmFn kQmm[3][8][3];  // [log2 MB]: 64, 128 or 256 rows per workgroup
 
-extern const WideFn kWide[3][8][3];  // [log2(R / 4)]: 64, 128 or 256 rows per workgroup
+// rows x columns per workgroup: 64 x 128, 128 x 256, 256 x 256
+extern const WideFn kWide[3][8][3];
+
+extern const MoeWideFn kMoeWide[8][3];  // expert QMMs for many rows per expert
+int moe_wide_rows(int k);  // their rows per block
+void launch_moe_route16(const MoePlanParams& pp, const MoeGatherParams& gp, size_t lds, hipStream_t s);
 
 // xhat of `members` (suh, xhat) pairs of p in one launch.
 void launch_prologue(const PrologueParams& p, int members, hipStream_t s);
-// Sums the split-K partials of a kWide launch of 16*R rows per workgroup and
-// finishes its outputs.
-void launch_wide_reduce(const WideParams& p, int R, hipStream_t s);
+// The same for the QMM (more than 16 rows): the Hadamard by MFMA.
+void launch_prologue16(const PrologueParams& p, int members, hipStream_t s);
+// Sums the split-K partials of a kWide launch of 16*R rows x 32*NW columns per
+// workgroup and finishes its outputs.
+void launch_wide_reduce(const WideParams& p, int R, int NW, hipStream_t s);
 // values[i] = codeword(states[i], cb).
 void launch_codewords(const uint16_t* states, int64_t n, int cb, uint16_t* values, hipStream_t s);
 // packed[t][16k] = the trellis tile of states[t][256] (low k bits of each).

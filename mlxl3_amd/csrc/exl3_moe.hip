@@ -93,6 +93,29 @@ int moe_splits(const exl3_moe* h, int64_t slots, int block_rows, int k_in, int c
   return std::max(1, std::min(s, k_in / 128));
 }
 
+// Whether the grouped expert QMMs run as moe_wide_kernel: where its blocks (160
+// rows, 128 at K = 8) decode an expert's weights at most half as often as
+// moe_mm_kernel's 64-row blocks on the average rows per expert.  Measured (us, old ->
+// new; rows per expert): 128 experts top-8 K = 3, 2048x768: 62 264 -> 298, 125 451 ->
+// 376, 250 825 -> 739; 64 experts top-6 K = 4, 2048x1024: 56 168 -> 188, 188 406 -> 425;
+// 8 experts top-2: 64 80 -> 87, 250 132 -> 106, 1000 268 -> 242; 32 experts top-4 K = 5,
+// 3072x1536: 125 362 -> 264.  Its copies address the bank and the gathered rows with
+// 32-bit byte offsets, 16 bytes at a time.  Pinned split counts or block rows keep
+// moe_mm_kernel.  EXL3_MOE_WIDE=0/1 forces it off or on (tuning).
+bool moe_takes_wide(const exl3_moe* h, int64_t slots) {
+  const int64_t bank = std::max((int64_t)2 * h->experts * h->hidden / 8 * h->k * h->in,
+                                (int64_t)h->experts * h->in / 8 * h->k * h->hidden);
+  const int64_t rows = std::max(2 * slots * h->in, slots * h->hidden) * 2;
+  if (bank >= ((int64_t)1 << 32) || rows >= ((int64_t)1 << 32)) return false;
+  if (((uintptr_t)h->gu_trellis | (uintptr_t)h->down_trellis) & 15) return false;
+  // the gate's and up's sums borrow the slot outputs' buffer (f32 rows of `in`)
+  if (h->hidden > h->in || h->hidden / 128 > 65535) return false;
+  if (h->force_splits > 1 || getenv("EXL3_MOE_BLOCK_ROWS")) return false;
+  if (const char* env = getenv("EXL3_MOE_WIDE")) return atoi(env) != 0;
+  const int64_t avg = slots / h->experts, rows_wide = moe_wide_rows(h->k);
+  return avg > 64 && (avg + 63) / 64 >= 2 * ((avg + rows_wide - 1) / rows_wide);
+}
+
 // The small-row path (decode): up to this many routed slots run as two
 // launches, one workgroup row per slot (moe_dec_*_kernel), where the grouped
 // path's four launches cost more than the weight reuse it offers (C4 bank,
@@ -127,6 +150,7 @@ int moe_small_splits(const exl3_moe* h, int64_t slots, int k_in, int col_blocks,
 struct MoeLayout {
   size_t counts, rank, sorted, expert_count, table, counters, xgu, xd, z, partials, total;
   int max_blocks, ncounters, splits_gu, splits_down, block_rows;
+  int wide;                         // the expert QMMs of exl3_moe_wide.hpp
   int small, small_gu, small_down;  // small-row path and its split counts
 };
 
@@ -145,6 +169,8 @@ bool moe_layout(const exl3_moe* h, int64_t rows, MoeLayout& L) {
     const int v = atoi(env);
     if (v == 16 || v == 32 || v == 64) L.block_rows = v;
   }
+  L.wide = moe_takes_wide(h, slots);
+  if (L.wide) L.block_rows = moe_wide_rows(h->k);
   // each routed expert's last block may be partial: sum ceil(c_e/b) <=
   // slots/b + (experts routed) <= slots/b + min(E, slots).  The expert QMM
   // grids are sized by this bound, so a decode call (8 slots) launches the
@@ -154,8 +180,8 @@ bool moe_layout(const exl3_moe* h, int64_t rows, MoeLayout& L) {
   if (ncounters > INT32_MAX) return false;
   L.max_blocks = (int)max_blocks;
   L.ncounters = (int)ncounters;
-  L.splits_gu = moe_splits(h, slots, L.block_rows, h->in, h->hidden / 128);
-  L.splits_down = moe_splits(h, slots, L.block_rows, h->hidden, h->in / 128);
+  L.splits_gu = L.wide ? 1 : moe_splits(h, slots, L.block_rows, h->in, h->hidden / 128);
+  L.splits_down = L.wide ? 1 : moe_splits(h, slots, L.block_rows, h->hidden, h->in / 128);
   // small-row path: its arrival counters (gate/up, down, top-k sums) must fit
   // the workspace's counter region
   const int64_t small_counters =
@@ -365,9 +391,9 @@ int exl3_moe_forward(const exl3_moe* h, const void* x, int32_t x_type, int64_t r
   const int mbi = L.block_rows == kMoeMaxBlockRows ? 2 : L.block_rows == 32 ? 1 : 0;
   const MoeKernel gateup = kGateUp[mbi][h->k - 1][h->cb], down = kDown[mbi][h->k - 1][h->cb];
   if (!gateup || !down) return fail(EXL3_EUNSUPPORTED, "no SwitchGLU kernel for K=%d", h->k);
-  const int64_t wide = (int64_t)(L.max_blocks + 7) * (std::max(h->in, h->hidden) / 128) *
+  const int64_t grid_size = (int64_t)(L.max_blocks + 7) * (std::max(h->in, h->hidden) / 128) *
                        std::max(L.splits_gu, L.splits_down);
-  if (wide * 512 >= ((int64_t)1 << 31))
+  if (grid_size * 512 >= ((int64_t)1 << 31))
     return fail(EXL3_EUNSUPPORTED, "SwitchGLU launch of %lld rows is too large", (long long)rows);
   hipStream_t s = (hipStream_t)stream;
   char* ws = (char*)workspace;
@@ -401,7 +427,9 @@ int exl3_moe_forward(const exl3_moe* h, const void* x, int32_t x_type, int64_t r
       1u + (unsigned)((2 * (int64_t)slots * ((h->in / 128 + 7) / 8) + 3) / 4);
   const size_t plan_lds = (3 * (size_t)h->experts + 1) * sizeof(int);
   if (int rc = launch_gate("moe plan")) return rc;
-  if ((((uintptr_t)x | (uintptr_t)h->gu_suh) & 15) == 0)
+  if (L.wide)
+    launch_moe_route16(pp, gp, plan_lds, s);
+  else if ((((uintptr_t)x | (uintptr_t)h->gu_suh) & 15) == 0)
     moe_route_kernel<true><<<route_wgs, 256, plan_lds, s>>>(pp, gp);
   else
     moe_route_kernel<false><<<route_wgs, 256, plan_lds, s>>>(pp, gp);
@@ -444,9 +472,15 @@ int exl3_moe_forward(const exl3_moe* h, const void* x, int32_t x_type, int64_t r
   d.scores = scores;
   d.scores_dtype = scores_type;
   d.z = ws + L.z;
-  gateup<<<grid_blocks * q.col_blocks * q.splits, 512, 0, s>>>(q);
+  if (L.wide)
+    kMoeWide[h->k - 1][h->cb](q, true, grid_blocks, (uint16_t*)d.z, s);
+  else
+    gateup<<<grid_blocks * q.col_blocks * q.splits, 512, 0, s>>>(q);
   if (int rc = check_launch("moe gate/up")) return rc;
-  down<<<grid_blocks * d.col_blocks * d.splits, 256, 0, s>>>(d);
+  if (L.wide)
+    kMoeWide[h->k - 1][h->cb](d, false, grid_blocks, nullptr, s);
+  else
+    down<<<grid_blocks * d.col_blocks * d.splits, 256, 0, s>>>(d);
   if (int rc = check_launch("moe down")) return rc;
 
   const dim3 rgrid((unsigned)rows, (h->in + 2047) / 2048);

@@ -623,7 +623,7 @@ __attribute__((amdgpu_waves_per_eu(MB == 4 ? 2 : CB == 2 ? 3 : 4))) void moe_mm_
 // moe_finish_row on f32 gate/up rows [2s], [2s+1] of slot s.  One wave per
 // (slot, 128-column block); grid (slots, hidden / 128).  Slots routed to an
 // expert id >= experts get zeros (the reference reads out of its bank).
-__global__ __launch_bounds__(64) void swiglu_down_input_kernel(MoeMmParams p,
+static __global__ __launch_bounds__(64) void swiglu_down_input_kernel(MoeMmParams p,
                                                                const float* __restrict__ gate_up,
                                                                const uint32_t* selected) {
   const int slot = blockIdx.x, cblk = blockIdx.y, lane = threadIdx.x;
@@ -643,7 +643,7 @@ __global__ __launch_bounds__(64) void swiglu_down_input_kernel(MoeMmParams p,
 // (f32 adds), rounded to f16 for f16 scores; H the staged Hadamard with
 // f16(v * scale), svh one row per slot.  One wave per (row, 128-column block);
 // grid (rows, width / 128).
-__global__ __launch_bounds__(64) void finish_and_reduce_kernel(const float* __restrict__ raw,
+static __global__ __launch_bounds__(64) void finish_and_reduce_kernel(const float* __restrict__ raw,
                                                                const uint16_t* __restrict__ svh,
                                                                const void* __restrict__ scores,
                                                                int scores_dtype, int top_k,

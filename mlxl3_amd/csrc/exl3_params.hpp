@@ -57,23 +57,23 @@ struct QmmParams {
   int splits;          // K-ranges per output tile (global split-K)
 };
 
-// A projection of a wide QMM launch: it owns the column pairs (256 columns)
-// [pair0, pair0 + ceil(out / 256)).
+// A projection of a wide QMM launch: it owns the column units (128 or 256 columns)
+// [unit0, unit0 + ceil(out / columns)).
 struct WideMember {
   const uint32_t* trellis;
   const uint16_t* xhat;  // [M][in] f16
   const uint16_t* svh;
   const uint16_t* bias;
   void* y;
-  int out, pair0, y_dtype;
+  int out, unit0, y_dtype;
 };
 struct WideParams {
   WideMember mem[kMaxMembers];
   int members;
-  float* partials;     // [splits][tiles][16*R x 256 f32 in fragment order] (splits > 1)
+  float* partials;     // [splits][tiles][16*R x 32*NW f32 in fragment order] (splits > 1)
   uint32_t* counters;  // [mtiles * pairs], zero between calls (splits > 1)
   int in, M, x_dtype;
-  int pairs;   // column pairs of all members
+  int units;   // column units of all members
   int mtiles;  // ceil(M / rows per workgroup)
   int splits;
 };
@@ -99,11 +99,11 @@ __device__ __forceinline__ Member select_member(const P& p, int cblk) {
 }
 
 template <typename P>
-__device__ __forceinline__ WideMember select_wide(const P& p, int pair) {
+__device__ __forceinline__ WideMember select_wide(const P& p, int unit) {
   WideMember m = p.mem[0];
 #pragma unroll
   for (int i = 1; i < kMaxMembers; ++i)
-    if (i < p.members && pair >= p.mem[i].pair0) m = p.mem[i];
+    if (i < p.members && unit >= p.mem[i].unit0) m = p.mem[i];
   return m;
 }
 

@@ -13,6 +13,8 @@ namespace exl3 {
 EXL3_INSTANTIATE(EXL3_QMM_INST)
 template __global__ void prologue_kernel<true>(PrologueParams);
 template __global__ void prologue_kernel<false>(PrologueParams);
+template __global__ void prologue16_kernel<true>(PrologueParams);
+template __global__ void prologue16_kernel<false>(PrologueParams);
 template __global__ void swiglu_prepare_kernel<true>(const uint16_t*, const uint16_t*,
                                                      const uint16_t*, int, int, uint16_t*);
 template __global__ void swiglu_prepare_kernel<false>(const uint16_t*, const uint16_t*,
@@ -93,6 +95,17 @@ void launch_prologue(const PrologueParams& p, int members, hipStream_t s) {
                        dim3(256), 0, s, p);
 }
 
+void launch_prologue16(const PrologueParams& p, int members, hipStream_t s) {
+  const int64_t groups = ((int64_t)((p.rows + 15) / 16) * (p.in / 128) + 3) / 4;
+  uintptr_t bits = (uintptr_t)p.x;
+  for (int i = 0; i < members; ++i) bits |= (uintptr_t)p.suh[i] | (uintptr_t)p.xhat[i];
+  const dim3 grid((unsigned)groups, (unsigned)members);
+  if ((bits & 15) == 0)
+    hipLaunchKernelGGL(prologue16_kernel<true>, grid, dim3(256), 0, s, p);
+  else
+    hipLaunchKernelGGL(prologue16_kernel<false>, grid, dim3(256), 0, s, p);
+}
+
 void launch_glu(const uint16_t* gate, const uint16_t* up, uint16_t* out, int64_t n, bool gelu,
                 hipStream_t s) {
   const int vec = ((((uintptr_t)gate | (uintptr_t)up | (uintptr_t)out) & 15) == 0) ? 1 : 0;
@@ -106,7 +119,7 @@ void launch_glu(const uint16_t* gate, const uint16_t* up, uint16_t* out, int64_t
 
 void launch_swiglu_prepare(const uint16_t* gate, const uint16_t* up, const uint16_t* down_suh,
                            int H, int rows, uint16_t* xhat, hipStream_t s) {
-  const unsigned groups = (unsigned)(((int64_t)rows * (H / 128) + 15) / 16);
+  const unsigned groups = (unsigned)(((int64_t)((rows + 15) / 16) * (H / 128) + 3) / 4);
   if ((((uintptr_t)gate | (uintptr_t)up | (uintptr_t)down_suh | (uintptr_t)xhat) & 15) == 0)
     hipLaunchKernelGGL(swiglu_prepare_kernel<true>, dim3(groups), dim3(256), 0, s, gate, up,
                        down_suh, H, rows, xhat);

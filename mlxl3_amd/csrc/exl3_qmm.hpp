@@ -74,43 +74,6 @@ __global__ __launch_bounds__(256) void prologue_kernel(PrologueParams p) {
                  xhat + e, live, threadIdx.x & 63);
 }
 
-// The SwiGLU edge between a (gate, up) group and its down projection:
-// xhat_down = f16(H128(f16(swiglu(g, u) * down_suh)) / sqrt(128)) (the down
-// projection's prologue applied to the activation, as the reference's
-// flash_up_finish_swiglu_prepare fuses them, exl3.metal:265-291, with
-// Array::swiglu's f16 arithmetic).  16 lanes per (row, 128-block) job, 8
-// columns per lane (finish8).  grid (ceil(rows * H / 128 / 16)), 256 threads.
-template <bool VEC>
-__global__ __launch_bounds__(256) void swiglu_prepare_kernel(const uint16_t* __restrict__ gate,
-                                                             const uint16_t* __restrict__ up,
-                                                             const uint16_t* __restrict__ down_suh,
-                                                             int H, int rows,
-                                                             uint16_t* __restrict__ xhat) {
-  int row, b;
-  const bool live = job16(rows, H >> 7, row, b);
-  const int c = b * 128 + 8 * (threadIdx.x & 15);
-  const size_t e = (size_t)row * H + c;
-  float a[8], sv[8];
-  if constexpr (VEC) {
-    const u32x4 gw = *(const u32x4*)(gate + e), uw = *(const u32x4*)(up + e);
-    const u32x4 sw = *(const u32x4*)(down_suh + c);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      a[2 * i] = swiglu_f16(h2f((uint16_t)gw[i]), h2f((uint16_t)uw[i]));
-      a[2 * i + 1] = swiglu_f16(h2f((uint16_t)(gw[i] >> 16)), h2f((uint16_t)(uw[i] >> 16)));
-      sv[2 * i] = h2f((uint16_t)sw[i]);
-      sv[2 * i + 1] = h2f((uint16_t)(sw[i] >> 16));
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      a[i] = swiglu_f16(h2f(gate[e + i]), h2f(up[e + i]));
-      sv[i] = h2f(down_suh[c + i]);
-    }
-  }
-  finish8<VEC>(a, sv, xhat + e, live, threadIdx.x & 63);
-}
-
 // Rows of a finished tile pass through LDS as f16: Y[row][136] (128 columns
 // plus 8 halves of padding: the 8-byte reads of 16 rows then touch every bank
 // once).  The columns of a 16-column tile sit at position 2*(c % 8) + c / 8, which
@@ -125,6 +88,191 @@ typedef float float2v __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ half2v pack_f16(float a, float b) {
   return __builtin_convertvector(float2v{a, b}, half2v);
 }
+
+// The Hadamard-128 of 16 rows held as 8 x 4 columns per lane (lane (g, n): columns
+// 16i + 4g + r of row n), without the 1/sqrt(128).  STAGED rounds to f16 after
+// strides 8 and 64.  in[i]: the lane's four columns of group i as MFMA operand;
+// hm: H16's row n at those columns.
+template <bool STAGED>
+__device__ __forceinline__ void h128_mfma(const half4 (&in)[8], half4 hm, float (&v)[8][4]) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float4v d =
+        __builtin_amdgcn_mfma_f32_16x16x16f16(hm, in[i], float4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[i][r] = STAGED ? round_f16(d[r]) : d[r];
+  }
+#pragma unroll
+  for (int s = 1; s < 8; s <<= 1)
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (!(i & s))
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float p = v[i][r], q = v[i + s][r];
+          v[i][r] = p + q;
+          v[i + s][r] = p - q;
+        }
+  if (STAGED) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[i][r] = round_f16(v[i][r]);
+  }
+}
+
+// H16's row n at columns 4g..4g+3, or at the columns of positions 4g..4g+3 of a
+// staged row (qmm_stage_row's order).
+template <bool POSITIONS>
+__device__ __forceinline__ half4 h16_row(int lane) {
+  const int g = lane >> 4, n = lane & 15;
+  half4 hm;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int c = POSITIONS ? 2 * g + (i >> 1) + 8 * (i & 1) : 4 * g + i;
+    hm[i] = (__builtin_popcount(c & n) & 1) ? -1.f : 1.f;
+  }
+  return hm;
+}
+
+// f16(x * s) of eight consecutive inputs (f16(f16(x) * s), as finish8: the f32
+// product of two f16 values is exact, so its rounding is the f16 product).
+template <bool VEC>
+__device__ __forceinline__ half8 scaled8(const void* x, int x_dtype, size_t xe, const uint16_t* s) {
+  half8 a, sv;
+  if constexpr (VEC) {
+    sv = *(const half8*)s;
+    if (x_dtype == DT_F16) return *(const half8*)((const uint16_t*)x + xe) * sv;
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sv[i] = __builtin_bit_cast(_Float16, s[i]);
+  }
+  float f[8];
+  load8_act<VEC>(x, x_dtype, xe, f);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) a[i] = (_Float16)f[i];
+  return a * sv;
+}
+
+// f16(H128(.) / sqrt(128)) of 16 rows x 128 columns by one wave: lane l gives and
+// gets the 8 columns 8*(l % 16).. of rows 4t + l / 16 (t = 0..3), 16 bytes each, so
+// that rows come and go as whole 256-byte lines; the transform's own layout
+// (h128_mfma) is reached through the wave's LDS (its own accesses, in order).
+// Loading and storing that layout directly, 32 bytes per row and instruction, took
+// 20.9 us for 2048 x 4096 inputs x 2 members.
+__device__ __forceinline__ void h128_rows16(half8 (&io)[4], uint16_t* ys, int lane) {
+  const int g = lane >> 4, n = lane & 15;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) *(half8*)(ys + (4 * t + g) * kYStride + 8 * n) = io[t];
+  half4 in[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) in[i] = *(const half4*)(ys + n * kYStride + 16 * i + 4 * g);
+  float v[8][4];
+  h128_mfma<true>(in, h16_row<false>(lane), v);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const half2v lo = pack_f16(v[i][0] * kHadScale, v[i][1] * kHadScale);
+    const half2v hi = pack_f16(v[i][2] * kHadScale, v[i][3] * kHadScale);
+    *(half4*)(ys + n * kYStride + 16 * i + 4 * g) = half4{lo[0], lo[1], hi[0], hi[1]};
+  }
+#pragma unroll
+  for (int t = 0; t < 4; ++t) io[t] = *(const half8*)(ys + (4 * t + g) * kYStride + 8 * n);
+}
+
+template <bool VEC>
+__device__ __forceinline__ void store8(half8 v, uint16_t* dst) {
+  if constexpr (VEC) {
+    *(half8*)dst = v;
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) dst[i] = __builtin_bit_cast(uint16_t, v[i]);
+  }
+}
+
+// The QMM's prologue: prologue_kernel's values with the Hadamard by MFMA, one wave
+// per 16 rows x 128 columns (~30 -> ~9 VALU instructions per element).  Only for
+// more than 16 rows: the MFMA's f32 sums may round otherwise than the butterflies'
+// in rare cases, and a row of the QMV has one value whichever launch computes it.
+// grid (ceil(ceil(rows / 16) * blocks / 4), members), 256 threads.
+template <bool VEC>
+__global__ __launch_bounds__(256) void prologue16_kernel(PrologueParams p) {
+  __shared__ __attribute__((aligned(16))) uint16_t ys[4][16 * kYStride];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int job = blockIdx.x * 4 + wave;
+  const int nb = p.in >> 7, rg = job / nb, b = job - rg * nb;
+  if (16 * rg >= p.rows) return;  // uniform per wave
+  const uint16_t* suh = p.suh[0];
+  uint16_t* xhat = p.xhat[0];
+#pragma unroll
+  for (int i = 1; i < kMaxMembers; ++i)
+    if ((int)blockIdx.y == i) {
+      suh = p.suh[i];
+      xhat = p.xhat[i];
+    }
+  const int row0 = 16 * rg + (lane >> 4);
+  const size_t c0 = (size_t)b * 128 + 8 * (lane & 15);
+  half8 io[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+    io[t] = scaled8<VEC>(p.x, p.x_dtype, (size_t)min(row0 + 4 * t, p.rows - 1) * p.in + c0, suh + c0);
+  h128_rows16(io, ys[wave], lane);
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+    if (row0 + 4 * t < p.rows) store8<VEC>(io[t], xhat + (size_t)(row0 + 4 * t) * p.in + c0);
+}
+
+// The SwiGLU edge between a (gate, up) group and its down projection:
+// xhat_down = f16(H128(f16(swiglu(g, u) * down_suh)) / sqrt(128)) (the down
+// projection's prologue applied to the activation, as the reference's
+// flash_up_finish_swiglu_prepare fuses them, exl3.metal:265-291, with
+// Array::swiglu's f16 arithmetic), the Hadamard as in prologue16_kernel.  grid
+// (ceil(ceil(rows / 16) * H / 128 / 4)), 256 threads.
+template <bool VEC>
+__global__ __launch_bounds__(256) void swiglu_prepare_kernel(const uint16_t* __restrict__ gate,
+                                                             const uint16_t* __restrict__ up,
+                                                             const uint16_t* __restrict__ down_suh,
+                                                             int H, int rows,
+                                                             uint16_t* __restrict__ xhat) {
+  __shared__ __attribute__((aligned(16))) uint16_t ys[4][16 * kYStride];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int job = blockIdx.x * 4 + wave;
+  const int nb = H >> 7, rg = job / nb, b = job - rg * nb;
+  if (16 * rg >= rows) return;  // uniform per wave
+  const int row0 = 16 * rg + (lane >> 4);
+  const int c0 = b * 128 + 8 * (lane & 15);
+  half8 io[4], sv;
+  if constexpr (VEC) {
+    sv = *(const half8*)(down_suh + c0);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sv[i] = __builtin_bit_cast(_Float16, down_suh[c0 + i]);
+  }
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const size_t e = (size_t)min(row0 + 4 * t, rows - 1) * H + c0;
+    half8 gv, uv;
+    if constexpr (VEC) {
+      gv = *(const half8*)(gate + e);
+      uv = *(const half8*)(up + e);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        gv[i] = __builtin_bit_cast(_Float16, gate[e + i]);
+        uv[i] = __builtin_bit_cast(_Float16, up[e + i]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) io[t][i] = (_Float16)swiglu_f16((float)gv[i], (float)uv[i]);
+    io[t] = io[t] * sv;
+  }
+  h128_rows16(io, ys[wave], lane);
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+    if (row0 + 4 * t < rows) store8<VEC>(io[t], xhat + (size_t)(row0 + 4 * t) * H + c0);
+}
+
 
 // Consumer side: f16(acc) of one row into Y.  Register f of the lane holds
 // column 32*(f>>1) + 8*(f&1) + 16*(n>>3) + (n&7), n = lane & 15.
@@ -163,12 +311,14 @@ struct QmmOut {
 // each half as the staged transform has it.  Lane (g, n) ends with columns 16i +
 // 4g + 0..3 of row n.  ~9 VALU instructions per value, where the transform by
 // lane exchanges takes ~30.
-// RN = 2: only columns 4g + r0, r0 + 1 of each 4 (two waves share the rows).
+// 16-bit results go back to the staged rows' LDS (which no other wave uses) and
+// out as whole 256-byte lines.  RN = 2: only columns 4g + r0, r0 + 1 of each 4 (two
+// waves share the rows, and store directly).
 template <int RN = 4>
-__device__ __forceinline__ void qmm_finish16(const uint16_t* ys, int stride, const uint16_t* svh,
-                                             const uint16_t* bias, int lane, bool live,
+__device__ __forceinline__ void qmm_finish16(uint16_t* ys, int stride, const uint16_t* svh,
+                                             const uint16_t* bias, int lane, int rows,
                                              const QmmOut& out, int x_dtype, size_t yoff,
-                                             int r0 = 0) {
+                                             size_t ystride, int r0 = 0) {
   const int g = lane >> 4, n = lane & 15;
   half4 hm;  // H16 row n at the true columns of positions 4g + i
 #pragma unroll
@@ -213,7 +363,6 @@ __device__ __forceinline__ void qmm_finish16(const uint16_t* ys, int stride, con
       o[r] = pack_f16((float)h[0] * kHadScale, (float)h[1] * kHadScale) *
              *(const half2v*)(svh + c + 2 * r);
     }
-    if (!live) continue;
     uint32_t w[RN / 2];
     if (plain) {
 #pragma unroll
@@ -224,22 +373,32 @@ __device__ __forceinline__ void qmm_finish16(const uint16_t* ys, int stride, con
       for (int r = 0; r < RN; ++r)
         f[r] = out_cast((float)o[r >> 1][r & 1], h2f(bias[c + r]), out.has_bias, x_dtype);
       if (out.y_dtype == DT_F32) {
-        float* y = (float*)out.y + yoff + c;
-        if constexpr (RN == 4)
-          *(float4v*)y = float4v{f[0], f[1], f[2], f[3]};
-        else
-          *(float2v*)y = float2v{f[0], f[1]};
+        float* y = (float*)out.y + yoff + n * ystride + c;
+        if (n < rows) {
+          if constexpr (RN == 4)
+            *(float4v*)y = float4v{f[0], f[1], f[2], f[3]};
+          else
+            *(float2v*)y = float2v{f[0], f[1]};
+        }
         continue;
       }
 #pragma unroll
       for (int r = 0; r < RN / 2; ++r)
         w[r] = out16(f[2 * r], out.y_dtype) | (out16(f[2 * r + 1], out.y_dtype) << 16);
     }
-    uint16_t* y = (uint16_t*)out.y + yoff + c;
     if constexpr (RN == 4)
-      *(u32x2*)y = u32x2{w[0], w[1]};
-    else
-      *(uint32_t*)y = w[0];
+      *(u32x2*)(ys + n * stride + c) = u32x2{w[0], w[1]};
+    else if (n < rows)
+      *(uint32_t*)((uint16_t*)out.y + yoff + n * ystride + c) = w[0];
+  }
+  if constexpr (RN == 4) {
+    if (out.y_dtype == DT_F32) return;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int row = 4 * t + g;
+      const u32x4 w = *(const u32x4*)(ys + row * stride + 8 * n);
+      if (row < rows) *(u32x4*)((uint16_t*)out.y + yoff + row * ystride + 8 * n) = w;
+    }
   }
 }
 
@@ -658,9 +817,9 @@ __global__ __launch_bounds__(512) void qmm_kernel(QmmParams p) {
   const QmmOut out{mm.y, mm.y_dtype, mm.bias != nullptr};
   constexpr int kShare = MB == 1 ? 2 : 1;
   for (int u = wave / kShare; u < 4 * MB; u += 8 / kShare) {
-    const int row = mtile * 64 * MB + 16 * u + n;
-    qmm_finish16<4 / kShare>(ys + 16 * u * kYStride, kYStride, s_svh, s_bias, lane, row < p.M, out,
-                             p.x_dtype, (size_t)row * mm.out + cblk_l * 128,
+    const int row = mtile * 64 * MB + 16 * u;
+    qmm_finish16<4 / kShare>(ys + 16 * u * kYStride, kYStride, s_svh, s_bias, lane, p.M - row, out,
+                             p.x_dtype, (size_t)row * mm.out + cblk_l * 128, mm.out,
                              kShare == 2 ? 2 * (wave & 1) : 0);
   }
 }

@@ -1,4 +1,4 @@
-// The decode-in-registers QMM loop: 8 waves, 16*R rows x 256 columns, one
+// The decode-in-registers QMM loop: NW waves, 16*R rows x 32*NW columns, one
 // K-range, for the linear at more than 16 rows (qmm_tensor,
 // linear.rs:1874-2083).
 //
@@ -7,7 +7,7 @@
 // weight never passes through LDS and is decoded once per 16*R rows.  Everything
 // that comes from memory goes global -> LDS directly, into two rings of one slot
 // per step of 64 inputs: the A rows (xhat, one 128-byte line per row, swizzled)
-// and the trellis words of the step's 4 tile rows x 16 tiles.  In step q a wave
+// and the trellis words of the step's 4 tile rows x 2*NW tiles.  In step q a wave
 //   * issues the copies of steps q + SA - 1 (A) and q + SW - 1 (trellis),
 //   * decodes the trellis words of step q + 1 in pieces between the MFMAs, and
 //     reads those of step q + 2, and
@@ -34,25 +34,32 @@
 
 namespace exl3 {
 
-template <int K, int R>
+// NW waves, 32 * NW columns.
+template <int K, int R, int NW>
 struct WideShape {
-  static constexpr int kRows = 16 * R;
-  static constexpr int kA = kRows * 128, kW = 2048 * K;  // bytes of a ring's slot
+  static constexpr int kRows = 16 * R, kCols = 32 * NW;
+  static constexpr int kA = kRows * 128, kW = 256 * K * NW;  // bytes of a ring's slot
   static constexpr int kAJobs = kA / 1024, kWJobs = kW / 1024;  // 1 KB copies per step
-  static constexpr int PA = (kAJobs + 7) / 8, PW = (kWJobs + 7) / 8;  // per wave
-  // ring depths: up to 64 rows two workgroups share a CU
-  static constexpr int kBudget = R <= 4 ? 79 * 1024 : 158 * 1024;
-  static constexpr int SA = R >= 16 ? 3 : 4;
+  static constexpr int PA = (kAJobs + NW - 1) / NW, PW = (kWJobs + NW - 1) / NW;  // per wave
+  // ring depths: with 4 waves, and up to 64 rows, two workgroups share a CU
+  static constexpr int kBudget = NW == 4 || R <= 4 ? 79 * 1024 : 158 * 1024;
+  static constexpr int SA = 4 * (kA + kW) <= kBudget ? 4 : 3;
   static constexpr int kFitW = (kBudget - SA * kA) / kW;
   static constexpr int SW = kFitW < 3 ? 3 : kFitW > 6 ? 6 : kFitW;
-  // trellis words are read two steps ahead where the ring is deep enough
-  static constexpr int kLead = SW >= 4 ? 2 : 1;
-  // copies that may be outstanding at a step's end: step q + 2's A rows and step
-  // q + kLead + 1's trellis words must have landed
-  static constexpr int kOutA = PW + (SA - 3) * (PA + PW);
-  static constexpr int kOutW = (SW - kLead - 2) * (PA + PW);
-  static constexpr int kOut = kOutA < kOutW ? kOutA : kOutW;
-  static constexpr int kY = kRows * 264 * 2;  // the tile's f16 rows (kWideStride)
+  // kAhead: the first A fragments of a step are read in the step before, which
+  // costs a ring slot (the copy has one step less to land in)
+  static constexpr bool kAhead = SA >= 4;
+  // trellis words are read two steps ahead (else one) where the ring is deep enough
+  static constexpr int kLead = SW >= 5 ? 2 : 1;
+  // copies that may be outstanding at a step's end where a wave issues pa A copies
+  // per step: what the next step reads must have landed, A of step q + 1 (+ 1 with
+  // kAhead) and trellis of step q + 1 + kLead
+  static constexpr int out(int pa) {
+    const int a = PW + (SA - (kAhead ? 3 : 2)) * (pa + PW), w = (SW - kLead - 2) * (pa + PW);
+    return a < w ? a : w;
+  }
+  static constexpr int kStride = kCols + 8;  // halves per staged output row
+  static constexpr int kY = kRows * kStride * 2;
   static constexpr int kRings = SA * kA + SW * kW;
   static constexpr int kLds = kRings > kY ? kRings : kY;
 };
@@ -224,32 +231,43 @@ constexpr int kDecodePieces = 34;
 // acc[rb][cg] += A (16*R rows) x this wave's 32 columns over nq steps.  lds: the
 // rings; aoff, woff: the lane's byte offset of each of the wave's copies in its
 // source.  Register r of lane (g = lane / 16, n = lane % 16) of acc[rb][cg] is row
-// 16rb + 4g + r, column 16*(n / 8) + n % 8 + 8cg of the wave's 32.
-template <int K, int CB, int R>
+// 16rb + 4g + r, column 16*(n / 8) + n % 8 + 8cg of the wave's 32.  With SOME, only
+// the first `live` row blocks (uniform, 1..R) are copied and, rounded up to a pair,
+// multiplied.
+template <int K, int CB, int R, int NW, bool SOME>
 __device__ __forceinline__ void wide_mm(uint8_t* lds, const WideSource& asrc, const WideSource& wsrc,
-                                        const uint32_t (&aoff)[WideShape<K, R>::PA],
-                                        const uint32_t (&woff)[WideShape<K, R>::PW], int nq, int wave,
-                                        int lane, float4v (&acc)[R][2]) {
-  using C = WideShape<K, R>;
-  constexpr int kRing = R >= 16 || R <= 4 ? 2 : 4;  // slot pairs of A fragments in registers
+                                        const uint32_t (&aoff)[WideShape<K, R, NW>::PA],
+                                        const uint32_t (&woff)[WideShape<K, R, NW>::PW], int nq,
+                                        int live, int wave, int lane, float4v (&acc)[R][2]) {
+  using C = WideShape<K, R, NW>;
+  constexpr int kRing = R == 8 ? 4 : 2;  // slot pairs of A fragments in registers
   const int g = lane >> 4, am = lane & 15, hsel = (lane >> 3) & 1, j = lane & 7;
   const uint32_t lds0 = lds_offset(lds);
-  // copy i of the wave is the step's copy wave + 8 * i; past the last one it
+  // copy i of the wave is the step's copy wave + NW * i; past the last one it
   // repeats that
+  const int ajobs = SOME ? 2 * live : C::kAJobs;
+  const int pa = SOME ? (max(ajobs - wave, 0) + NW - 1) / NW : C::PA;  // A copies per step
+  auto wait_copies = [&]() {
+    static_for<C::PA + 1>([&](auto pa_) {
+      constexpr int n = decltype(pa_)::value;
+      if (SOME ? pa == n : n == C::PA) __builtin_amdgcn_s_waitcnt(vmcnt_only(C::out(n)));
+    });
+  };
   uint32_t alds[C::PA], wlds[C::PW];
 #pragma unroll
   for (int i = 0; i < C::PA; ++i)
-    alds[i] = __builtin_amdgcn_readfirstlane(lds0 + min(wave + 8 * i, C::kAJobs - 1) * 1024);
+    alds[i] = __builtin_amdgcn_readfirstlane(lds0 + min(wave + NW * i, C::kAJobs - 1) * 1024);
 #pragma unroll
   for (int i = 0; i < C::PW; ++i)
     wlds[i] = __builtin_amdgcn_readfirstlane(lds0 + C::SA * C::kA +
-                                             min(wave + 8 * i, C::kWJobs - 1) * 1024);
+                                             min(wave + NW * i, C::kWJobs - 1) * 1024);
   const uint32_t a_end = (uint32_t)(nq - 1) * asrc.step, w_end = (uint32_t)(nq - 1) * wsrc.step;
   uint32_t a_at = 0, w_at = 0;  // byte offsets of the next step to copy
   // past the end: the last step again, into a slot that is not read
   auto copy_a = [&](uint32_t slot) {
 #pragma unroll
-    for (int i = 0; i < C::PA; ++i) wide_copy(asrc.rsrc, aoff[i], a_at, slot, alds[i]);
+    for (int i = 0; i < C::PA; ++i)
+      if (!SOME || wave + NW * i < ajobs) wide_copy(asrc.rsrc, aoff[i], a_at, slot, alds[i]);
     a_at = min(a_at + asrc.step, a_end);
   };
   auto copy_w = [&](uint32_t slot) {
@@ -261,19 +279,25 @@ __device__ __forceinline__ void wide_mm(uint8_t* lds, const WideSource& asrc, co
   // swizzle depends on the row's low 4 bits only)
   int foff[2];
 #pragma unroll
-  for (int h = 0; h < 2; ++h) foff[h] = am * 128 + (((2 * g + h) ^ a_swizzle(am)) << 4);
+  for (int h = 0; h < 2; ++h)
+    foff[h] = am * 128 + (((2 * g + h) ^ a_swizzle(am)) << 4);
   auto read_a = [&](half8& dst, uint32_t at, auto slot_) {
     constexpr int slot = decltype(slot_)::value, h = slot / R, rb = slot % R;
     dst = *(const half8*)(lds + at + foff[h] + rb * 2048);
   };
   // both fragments of slot pair `pr`; the first one used is read last, so one
   // wait serves both
+  auto pair_live = [&](auto pr_) {
+    constexpr int rb = 2 * decltype(pr_)::value % R;
+    return !SOME || rb == 0 || rb < live;
+  };
   auto read_pair = [&](half8(&dst)[2], uint32_t at, auto pr_) {
     constexpr int pr = decltype(pr_)::value;
+    if (!pair_live(pr_)) return;
     read_a(dst[1], at, std::integral_constant<int, 2 * pr + 1>{});
     read_a(dst[0], at, std::integral_constant<int, 2 * pr>{});
   };
-  const int wbase = C::SA * C::kA + ((g * 16 + 2 * wave + hsel) * 8 * K + j * K) * 4;
+  const int wbase = C::SA * C::kA + ((g * 2 * NW + 2 * wave + hsel) * 8 * K + j * K) * 4;
   const int wprev = wbase + (j == 0 ? 8 * K - 1 : -1) * 4;
   auto read_w = [&](uint32_t(&w)[K + 1], uint32_t at) {
     w[0] = *(const uint32_t*)(lds + at + wprev);
@@ -301,7 +325,7 @@ __device__ __forceinline__ void wide_mm(uint8_t* lds, const WideSource& asrc, co
     if (i + C::SA - 1 >= 0) copy_a((i + C::SA - 1) * C::kA);
     if (i + C::SW - 1 >= 0) copy_w((i + C::SW - 1) * C::kW);
   }
-  __builtin_amdgcn_s_waitcnt(vmcnt_only(C::kOut));
+  wait_copies();
   __syncthreads();
 
   u32x4 b[2][4] = {};
@@ -312,7 +336,8 @@ __device__ __forceinline__ void wide_mm(uint8_t* lds, const WideSource& asrc, co
     read_w(w[0], 0);
     static_for<kDecodePieces>([&](auto i) { dec.template piece<decltype(i)::value>(w[0], z, b[0]); });
     if (C::kLead == 2) read_w(w[0], C::kW);
-    static_for<kRing>([&](auto i) { read_pair(a[decltype(i)::value], 0, i); });
+    if (C::kAhead)
+      static_for<kRing>([&](auto i) { read_pair(a[decltype(i)::value], 0, i); });
   }
   // ring positions: A of steps q, q + 1 and q + SA - 1 (= q - 1), trellis of steps
   // q + kLead and q + SW - 1 (= q - 1)
@@ -325,32 +350,59 @@ __device__ __forceinline__ void wide_mm(uint8_t* lds, const WideSource& asrc, co
     constexpr int wi = C::kLead == 2 ? ph : 0;
     StepDecode<K, CB> dec;
     if (C::kLead == 1) read_w(w[0], wt);
+    if constexpr (!C::kAhead)
+      static_for<kRing>([&](auto i) { read_pair(a[decltype(i)::value], at, i); });
     u32x4(&cur)[4] = b[ph];
     u32x4(&nxt)[4] = b[ph ^ 1];
     // written by inline assembly: 2 wait states before the MFMAs
     asm volatile("s_nop 1" : "+v"(cur[0]), "+v"(cur[1]), "+v"(cur[2]), "+v"(cur[3]));
-    static_for<4 * R>([&](auto m_) {
-      constexpr int m = decltype(m_)::value, slot = m >> 1, cg = m & 1, h = slot / R, rb = slot % R;
-      constexpr int pr = slot >> 1;
-      acc[rb][cg] = mfma16(a[pr % kRing][slot & 1], __builtin_bit_cast(half8, cur[2 * h + cg]),
-                           acc[rb][cg]);
-      if constexpr (m % 4 == 3) {
+    // without fragments read ahead, some of the decode covers their latency
+    constexpr int kFirst = C::kAhead ? 0 : 4;
+    static_for<kFirst>([&](auto i) {
+      dec.template piece<decltype(i)::value>(w[wi], z, nxt);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    static_for<R>([&](auto pr_) {
+      constexpr int pr = decltype(pr_)::value;
+      auto pieces = [&](auto m_) {
+        constexpr int m = decltype(m_)::value;
+        constexpr int kRest = kDecodePieces - kFirst;
+        constexpr int i0 = kFirst + kRest * m / (4 * R), i1 = kFirst + kRest * (m + 1) / (4 * R);
+        static_for<i1 - i0>([&](auto i) {
+          dec.template piece<i0 + decltype(i)::value>(w[wi], z, nxt);
+        });
+      };
+      auto read_next = [&]() {
         if constexpr (pr + kRing < R)
           read_pair(a[pr % kRing], at, std::integral_constant<int, pr + kRing>{});
-        else
+        else if constexpr (C::kAhead)
           read_pair(a[pr % kRing], at1, std::integral_constant<int, pr + kRing - R>{});
+        if constexpr (C::kLead == 2 && pr == R / 2) read_w(w[wi ^ 1], wt);
+      };
+      if (pair_live(pr_)) {
+        static_for<4>([&](auto i_) {
+          constexpr int i = decltype(i_)::value, slot = 2 * pr + (i >> 1), cg = i & 1;
+          constexpr int h = slot / R, rb = slot % R;
+          acc[rb][cg] = mfma16(a[pr % kRing][slot & 1],
+                               __builtin_bit_cast(half8, cur[2 * h + cg]), acc[rb][cg]);
+          if constexpr (i == 3) read_next();
+          pieces(std::integral_constant<int, 4 * pr + i>{});
+          __builtin_amdgcn_sched_barrier(0);
+        });
+      } else {
+        // no rows: this pair's share of the decode alone, the compiler's own
+        // wait states between the pieces
+        read_next();
+        static_for<4>([&](auto i_) {
+          pieces(std::integral_constant<int, 4 * pr + decltype(i_)::value>{});
+          __builtin_amdgcn_sched_barrier(0);
+        });
       }
-      if constexpr (C::kLead == 2 && m == 2 * R) read_w(w[wi ^ 1], wt);
-      constexpr int i0 = kDecodePieces * m / (4 * R), i1 = kDecodePieces * (m + 1) / (4 * R);
-      static_for<i1 - i0>([&](auto i) {
-        dec.template piece<i0 + decltype(i)::value>(w[wi], z, nxt);
-      });
-      __builtin_amdgcn_sched_barrier(0);
     });
     // what the next step reads has landed; every wave is done with the slots that
     // the next step's copies overwrite, whose reads its MFMAs and decode have
     // waited for
-    __builtin_amdgcn_s_waitcnt(vmcnt_only(C::kOut));
+    wait_copies();
     asm volatile("s_barrier" ::: "memory");
     atd = at;
     at = at1;
@@ -369,60 +421,60 @@ __device__ __forceinline__ void wide_mm(uint8_t* lds, const WideSource& asrc, co
   __syncthreads();
 }
 
-constexpr int kWideStride = 264;  // halves per staged row of 256 columns
-
 // f16 rows of the tile in LDS from the accumulators of wide_mm.
 template <int R>
-__device__ __forceinline__ void wide_stage_rows(const float4v (&acc)[R][2], uint16_t* ys, int wave,
-                                                int lane) {
+__device__ __forceinline__ void wide_stage_rows(const float4v (&acc)[R][2], uint16_t* ys, int stride,
+                                                int wave, int lane) {
   const int g = lane >> 4, n = lane & 15;
-  uint16_t* y = ys + 4 * g * kWideStride + 32 * wave + 16 * (n >> 3) + 2 * (n & 7);
+  uint16_t* y = ys + 4 * g * stride + 32 * wave + 16 * (n >> 3) + 2 * (n & 7);
   static_for<R>([&](auto rb_) {
     constexpr int rb = decltype(rb_)::value;
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-      *(half2v*)(y + (16 * rb + r) * kWideStride) = pack_f16(acc[rb][0][r], acc[rb][1][r]);
+      *(half2v*)(y + (16 * rb + r) * stride) = pack_f16(acc[rb][0][r], acc[rb][1][r]);
   });
 }
 
-// Linear at more than 16 rows: tiles of 16*R rows x 256 columns of one member.
-template <int K, int CB, int R>
-__global__ __launch_bounds__(512) void wide_qmm_kernel(WideParams p) {
-  using C = WideShape<K, R>;
+// Linear at more than 16 rows: tiles of 16*R rows x 32*NW columns (a column unit)
+// of one member.
+template <int K, int CB, int R, int NW>
+__global__ __launch_bounds__(64 * NW) void wide_qmm_kernel(WideParams p) {
+  using C = WideShape<K, R, NW>;
   __shared__ __attribute__((aligned(16))) uint8_t lds[C::kLds];
-  __shared__ __attribute__((aligned(16))) uint16_t s_svh[256], s_bias[256];
+  __shared__ __attribute__((aligned(16))) uint16_t s_svh[C::kCols], s_bias[C::kCols];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
-  // Workgroup -> (row tile, column pair, split): each XCD takes a contiguous
-  // run, in which four row tiles of one column pair come together, so its L2
+  // Workgroup -> (row tile, column unit, split): each XCD takes a contiguous
+  // run, in which four row tiles of one column unit come together, so its L2
   // serves both the trellis (read once per four row tiles) and the A rows.
-  const int nwg = p.mtiles * p.pairs * p.splits;
+  const int nwg = p.mtiles * p.units * p.splits;
   const int id = blockIdx.x, xcd = id & 7, rem = nwg & 7;
   const int lin = xcd * (nwg >> 3) + min(xcd, rem) + (id >> 3);
-  const int per_split = p.mtiles * p.pairs;
+  const int per_split = p.mtiles * p.units;
   const int split = lin / per_split, in_split = lin - split * per_split;
-  const int band = in_split / (4 * p.pairs), in_band = in_split - band * 4 * p.pairs;
+  const int band = in_split / (4 * p.units), in_band = in_split - band * 4 * p.units;
   const int bh = min(4, p.mtiles - 4 * band);
-  const int pair = in_band / bh, mtile = 4 * band + (in_band - pair * bh);
-  const WideMember mm = select_wide(p, pair);
-  const int pl = pair - mm.pair0;  // column pair inside the member
+  const int unit = in_band / bh, mtile = 4 * band + (in_band - unit * bh);
+  const WideMember mm = select_wide(p, unit);
+  const int pl = unit - mm.unit0;  // column unit inside the member
   const int TN = mm.out >> 4;
-  const bool whole = pl * 256 + 128 < mm.out;  // the pair's second 128 columns exist
+  // the unit's second 128 columns exist
+  const bool whole = NW == 4 || pl * 256 + 128 < mm.out;
   const int nq_all = p.in >> 6;
   const int qa = split * nq_all / p.splits, nq = (split + 1) * nq_all / p.splits - qa;
-  const int tile = mtile * p.pairs + pair;
+  const int tile = mtile * p.units + unit;
   const int row0 = mtile * C::kRows;
 
-  if (threadIdx.x < 256) {
-    const int c = pl * 256 + (whole ? (int)threadIdx.x : (int)threadIdx.x & 127);
+  if (threadIdx.x < C::kCols) {
+    const int c = pl * C::kCols + (whole ? (int)threadIdx.x : (int)threadIdx.x & 127);
     s_svh[threadIdx.x] = mm.svh[c];
     s_bias[threadIdx.x] = mm.bias ? mm.bias[c] : 0;
   }
   const uint8_t* abase = (const uint8_t*)(mm.xhat + (size_t)row0 * p.in + (size_t)qa * 64);
   const WideSource asrc =
       wide_source(abase, (size_t)((const uint8_t*)(mm.xhat + (size_t)p.M * p.in) - abase), 128);
-  const size_t wfirst = ((size_t)4 * qa * TN + pl * 16) * (32 * K);
+  const size_t wfirst = ((size_t)4 * qa * TN + pl * 2 * NW) * (32 * K);
   const WideSource wsrc = wide_source((const uint8_t*)mm.trellis + wfirst,
                                       (size_t)(p.in >> 4) * TN * (32 * K) - wfirst,
                                       (uint32_t)TN * (128u * K));
@@ -431,45 +483,47 @@ __global__ __launch_bounds__(512) void wide_qmm_kernel(WideParams p) {
   for (int i = 0; i < C::PA; ++i) {
     // rows 8*jid..: lane l copies chunk (l & 7) ^ swizzle of row l >> 3; rows past
     // M repeat the last one (never stored)
-    const int r = 8 * min(wave + 8 * i, C::kAJobs - 1) + (lane >> 3);
+    const int r = 8 * min(wave + NW * i, C::kAJobs - 1) + (lane >> 3);
     const int rg = min(row0 + r, p.M - 1) - row0;
     aoff[i] = (uint32_t)((rg * p.in + ((lane & 7) ^ a_swizzle(r)) * 8) * 2);
   }
 #pragma unroll
   for (int i = 0; i < C::PW; ++i) {
-    // bytes v*1024 + 16*lane of the step's [4 tile rows][16 tiles]
-    const uint32_t at = (uint32_t)min(wave + 8 * i, C::kWJobs - 1) * 1024u + 16u * lane;
-    const uint32_t tr = at / (512u * K);
-    uint32_t rest = at - tr * (512u * K);
+    // bytes v*1024 + 16*lane of the step's [4 tile rows][2 * NW tiles]
+    const uint32_t at = (uint32_t)min(wave + NW * i, C::kWJobs - 1) * 1024u + 16u * lane;
+    const uint32_t tr = at / (64u * NW * K);
+    uint32_t rest = at - tr * (64u * NW * K);
     if (!whole && rest >= 256u * K) rest -= 256u * K;  // the missing half repeats the first
     woff[i] = tr * (uint32_t)TN * (32u * K) + rest;
   }
   float4v acc[R][2];
 #pragma unroll
   for (int rb = 0; rb < R; ++rb) acc[rb][0] = acc[rb][1] = float4v{0.f, 0.f, 0.f, 0.f};
-  wide_mm<K, CB, R>(lds, asrc, wsrc, aoff, woff, nq, wave, lane, acc);
+  wide_mm<K, CB, R, NW, false>(lds, asrc, wsrc, aoff, woff, nq, R, wave, lane, acc);
 
   if (p.splits > 1) {
     // split-K: the f32 sums, [split][tile][rb][wave][cg][lane] of 16 bytes, for
     // wide_reduce_kernel
-    float* slab = p.partials + ((size_t)split * per_split + tile) * (C::kRows * 256);
+    float* slab = p.partials + ((size_t)split * per_split + tile) * (C::kRows * C::kCols);
 #pragma unroll
     for (int rb = 0; rb < R; ++rb)
 #pragma unroll
       for (int cg = 0; cg < 2; ++cg)
-        *(float4v*)(slab + ((rb * 8 + wave) * 2 + cg) * 256 + lane * 4) = acc[rb][cg];
+        *(float4v*)(slab + ((rb * NW + wave) * 2 + cg) * 256 + lane * 4) = acc[rb][cg];
     return;
   }
   uint16_t* ys = (uint16_t*)lds;
-  wide_stage_rows<R>(acc, ys, wave, lane);
+  wide_stage_rows<R>(acc, ys, C::kStride, wave, lane);
   __syncthreads();
-  // R row blocks x two halves of 128 columns over the waves
+  // R row blocks x the unit's 128-column blocks over the waves
   const QmmOut out{mm.y, mm.y_dtype, mm.bias != nullptr};
-  for (int u = wave; u < 2 * R; u += 8) {
-    const int half = u & 1, rl = 16 * (u >> 1), row = row0 + rl + (lane & 15);
-    if ((half && !whole) || row0 + rl >= p.M) continue;  // uniform
-    qmm_finish16(ys + rl * kWideStride + 128 * half, kWideStride, s_svh + 128 * half, s_bias + 128 * half, lane,
-                row < p.M, out, p.x_dtype, (size_t)row * mm.out + pl * 256 + 128 * half);
+  constexpr int kH = NW / 4;
+  for (int u = wave; u < kH * R; u += NW) {
+    const int half = u % kH, rl = 16 * (u / kH), row = row0 + rl;
+    if ((half && !whole) || row >= p.M) continue;  // uniform
+    qmm_finish16(ys + rl * C::kStride + 128 * half, C::kStride, s_svh + 128 * half,
+                 s_bias + 128 * half, lane, p.M - row, out, p.x_dtype,
+                 (size_t)row * mm.out + pl * C::kCols + 128 * half, mm.out);
   }
 }
 
@@ -477,29 +531,29 @@ __global__ __launch_bounds__(512) void wide_qmm_kernel(WideParams p) {
 // columns adds the parts in split order.  A launch of its own: every CU takes
 // part and the partials go through the caches, where the last arriver of a tile
 // summing them alone (coherent loads, one workgroup per tile) was the larger
-// half of such calls.  grid ceil(mtiles * R * pairs * 2 / 4), 256 threads.
-static __global__ __launch_bounds__(256) void wide_reduce_kernel(WideParams p, int R) {
+// half of such calls.  grid ceil(mtiles * R * units * NW / 4 / 4), 256 threads.
+static __global__ __launch_bounds__(256) void wide_reduce_kernel(WideParams p, int R, int NW) {
   __shared__ __attribute__((aligned(16))) uint16_t ys[4][16 * kYStride];
   __shared__ __attribute__((aligned(16))) uint16_t s_svh[4][128], s_bias[4][128];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int tiles = p.mtiles * p.pairs;
-  const int unit = blockIdx.x * 4 + wave;
-  const int half = unit & 1, tr = unit >> 1;  // tr = tile * R + row block
+  const int tiles = p.mtiles * p.units;
+  const int kh = NW / 4, job = blockIdx.x * 4 + wave;
+  const int half = job % kh, tr = job / kh;  // tr = tile * R + row block
   const int tile = tr / R, rb = tr - tile * R;
-  const int mtile = tile / p.pairs, pair = tile - mtile * p.pairs;
+  const int mtile = tile / p.units, unit = tile - mtile * p.units;
   const int row0 = (mtile * R + rb) * 16;
   if (tile >= tiles || row0 >= p.M) return;  // uniform per wave
-  const WideMember mm = select_wide(p, pair);
-  const int col0 = (pair - mm.pair0) * 256 + 128 * half;
+  const WideMember mm = select_wide(p, unit);
+  const int col0 = (unit - mm.unit0) * 32 * NW + 128 * half;
   if (col0 >= mm.out) return;
 #pragma unroll
   for (int i = lane; i < 128; i += 64) {
     s_svh[wave][i] = mm.svh[col0 + i];
     s_bias[wave][i] = mm.bias ? mm.bias[col0 + i] : 0;
   }
-  const size_t slab = (size_t)R * 16 * 256, sstride = (size_t)tiles * slab;
-  const float* src = p.partials + (size_t)tile * slab + (rb * 8 + 4 * half) * 512 + lane * 4;
+  const size_t slab = (size_t)R * 16 * 32 * NW, sstride = (size_t)tiles * slab;
+  const float* src = p.partials + (size_t)tile * slab + (rb * NW + 4 * half) * 512 + lane * 4;
   float4v sum[8];
 #pragma unroll
   for (int f = 0; f < 8; ++f) sum[f] = *(const float4v*)(src + f * 256);
@@ -517,11 +571,10 @@ static __global__ __launch_bounds__(256) void wide_reduce_kernel(WideParams p, i
 #pragma unroll
     for (int r = 0; r < 4; ++r)
       *(half2v*)(y + r * kYStride + 32 * i) = pack_f16(sum[2 * i][r], sum[2 * i + 1][r]);
-  const int row = row0 + n;
   const QmmOut out{mm.y, mm.y_dtype, mm.bias != nullptr};
   // a wave's own rows: its LDS accesses stay in order
-  qmm_finish16(ys[wave], kYStride, s_svh[wave], s_bias[wave], lane, row < p.M, out, p.x_dtype,
-              (size_t)row * mm.out + col0);
+  qmm_finish16(ys[wave], kYStride, s_svh[wave], s_bias[wave], lane, p.M - row0, out, p.x_dtype,
+               (size_t)row0 * mm.out + col0, mm.out);
 }
 
 }  // namespace exl3

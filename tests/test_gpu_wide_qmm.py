@@ -1,6 +1,6 @@
-"""The decode-in-registers QMM (tiles of 64, 128 or 256 rows x 256 columns) at the
-edges of its tiles, forced on with EXL3_WIDE=1 and its shape with EXL3_WIDE_R /
-EXL3_WIDE_SPLITS, against the CPU oracle (tolerances of test_gpu_linear.py) and
+"""The decode-in-registers QMM (tiles of 64 rows x 128 columns, 128 x 256 or 256 x
+256) at the edges of its tiles, forced on with EXL3_WIDE=1 and its shape with
+EXL3_WIDE_TILE / EXL3_WIDE_SPLITS, against the CPU oracle (tolerances of test_gpu_linear.py) and
 against the producer/consumer QMM.
 
 One K-range on both sides multiplies and adds in the same order through the same
@@ -18,7 +18,7 @@ pytestmark = pytest.mark.gpu
 
 def force(monkeypatch, r, splits):
     monkeypatch.setenv("EXL3_WIDE", "1")
-    monkeypatch.setenv("EXL3_WIDE_R", str(r))
+    monkeypatch.setenv("EXL3_WIDE_TILE", str({4: 0, 8: 1, 16: 2}[r]))
     monkeypatch.setenv("EXL3_WIDE_SPLITS", str(splits))
     monkeypatch.setenv("EXL3_QMM_SPLITS", "1")  # read only where EXL3_WIDE=0
 
@@ -111,3 +111,52 @@ def test_workspace_between_the_two_needs(monkeypatch):
         check(y, ref, TOL_MODE1_REL, TOL_MODE1_ULP, f"workspace {size}")
     with pytest.raises(mlxl3_amd.Exl3Error, match="workspace too small"):
         lin.forward(t, workspace=torch.zeros(least - 256, dtype=torch.uint8, device="cuda"))
+
+
+# ---------------------------------------------------------------------------
+# the expert QMMs for many rows per expert
+# ---------------------------------------------------------------------------
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 6, 8])
+@pytest.mark.parametrize("cb", [0, 1, 2])
+def test_moe_wide_every_k_and_codebook(monkeypatch, k, cb):
+    """Experts whose rows fill one block, more than one and none, forced on."""
+    import test_gpu_moe as m
+
+    monkeypatch.setenv("EXL3_MOE_WIDE", "1")
+    print(f"moe wide k={k} cb={cb}", flush=True)
+    layer, x, _, _ = m.case(256, 128, 5, 2, 260, k, 700 + k)
+    sel, sc = synth.moe_routes(701 + k, 530, 260, 3, 2)  # ~173 rows each, experts 3 and 4 idle
+    moe = m.make_moe(layer, 2, k, cb)
+    pick = np.arange(0, 260, 7)
+    ref = oracle.moe_forward(x[pick], sel[pick], sc[pick], *layer, k, cb)
+    m.check(m.run(moe, x, sel, sc)[pick], ref, f"moe wide k={k} cb={cb}")
+
+
+@pytest.mark.parametrize("rows", [1, 8, 17, 80, 81, 161])
+@pytest.mark.parametrize("gelu", [False, True])
+@pytest.mark.parametrize("score", ["float16", "float32"])
+def test_moe_wide_rows(monkeypatch, rows, gelu, score):
+    """One expert takes every row (its block at and past its row blocks' edges),
+    with f16 and f32 scores, SiLU and GELU, and an id outside the bank."""
+    import test_gpu_moe as m
+
+    monkeypatch.setenv("EXL3_MOE_WIDE", "1")
+    print(f"moe wide rows={rows} gelu={gelu} {score}", flush=True)
+    layer, x, _, sc = m.case(384, 256, 3, 2, rows, 3, 720)
+    sel = np.tile(np.array([[1, 2]], np.uint32), (rows, 1))
+    sel[rows // 2:, 1] = 0
+    sel[0, 1] = 9  # outside: adds nothing
+    sc = sc.astype(score)
+    import torch
+    import mlxl3_amd
+
+    dev = lambda a: torch.from_numpy(a.view(np.int16) if a.dtype == np.uint16 else a).cuda()
+    moe = mlxl3_amd.Exl3SwitchGlu(*(dev(t) for t in layer), top_k=2, k=3, cb=0,
+                                  activation="gelu" if gelu else "silu",
+                                  logical_hidden=200 if gelu else None)
+    y = moe.forward(dev(x), torch.from_numpy(sel.astype(np.int32)).cuda(), dev(sc)).cpu().numpy()
+    monkeypatch.setenv("EXL3_MOE_WIDE", "0")
+    other = moe.forward(dev(x), torch.from_numpy(sel.astype(np.int32)).cuda(), dev(sc)).cpu().numpy()
+    # the grouped kernel is held to the oracle by test_gpu_moe.py; both sum the same
+    # products in the same order and differ by the epilogues' f32 sums
+    m.check(y, other, "vs the 64-row blocks")
