@@ -185,7 +185,10 @@ __device__ __forceinline__ void store8(half8 v, uint16_t* dst) {
     *(half8*)dst = v;
   } else {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) dst[i] = __builtin_bit_cast(uint16_t, v[i]);
+    for (int i = 0; i < 8; ++i) {
+      const _Float16 h = v[i];  // a bit cast of v[i] itself reads element 0 for every i
+      dst[i] = __builtin_bit_cast(uint16_t, h);
+    }
   }
 }
 

@@ -160,3 +160,22 @@ def test_moe_wide_rows(monkeypatch, rows, gelu, score):
     # the grouped kernel is held to the oracle by test_gpu_moe.py; both sum the same
     # products in the same order and differ by the epilogues' f32 sums
     m.check(y, other, "vs the 64-row blocks")
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16", "float32"])
+def test_moe_wide_unaligned_input(monkeypatch, dtype):
+    """An input one element past its alignment takes the gather's scalar loads and
+    gives the aligned input's bits."""
+    import test_gpu_moe as m
+    import torch
+
+    monkeypatch.setenv("EXL3_MOE_WIDE", "1")
+    print(f"moe wide unaligned {dtype}", flush=True)
+    layer, x, sel, sc = m.case(256, 128, 5, 2, 260, 3, 740)
+    moe = m.make_moe(layer, 2, 3, 0)
+    t = torch.from_numpy(x).cuda().to(getattr(torch, dtype))
+    buf = torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")[1:].view(t.shape).copy_(t)
+    sel, sc = torch.from_numpy(sel.astype(np.int32)).cuda(), torch.from_numpy(sc).cuda()
+    assert buf.data_ptr() % 16 != 0
+    a, b = moe.forward(t, sel, sc), moe.forward(buf, sel, sc)
+    assert torch.equal(a.float(), b.float())
