@@ -341,12 +341,12 @@ struct WideTile {
   double step_ns, alone_ns;   // a step with every CU full, and with one workgroup each
   double fixed_ns;            // ring fill, epilogue and output flush of a launch
 };
-static constexpr WideTile kWideTiles[3] = {{4, 4, 2, 1000, 750, 5000},
+static constexpr WideTile kWideTiles[3] = {{4, 4, 2, 1200, 750, 5000},
                                            {8, 8, 1, 1060, 1060, 9000},
                                            {16, 8, 1, 1560, 1560, 15000}};
 
-static size_t wide_partial_bytes(const WideTile& t, int64_t mtiles, int units, int splits) {
-  return splits > 1 ? sizeof(float) * (size_t)splits * mtiles * units * 16 * t.r * 32 * t.nw : 0;
+static size_t wide_partial_bytes(const WideTile& t, int64_t rows, int units, int splits) {
+  return splits > 1 ? sizeof(float) * (size_t)splits * ((rows + 15) / 16 * 16) * units * 32 * t.nw : 0;
 }
 
 // The cheapest shape whose partials fit in `budget` bytes (one split always fits);
@@ -365,7 +365,7 @@ static WideShape choose_wide_shape(int in, const int (&units)[2], int64_t rows, 
     for (int splits = 1; splits <= 8; ++splits) {
       int sp = force_splits ? force_splits : splits;
       sp = std::max(1, std::min(sp, std::max(1, nq / 4)));
-      const size_t part = wide_partial_bytes(t, mt, u, sp);
+      const size_t part = wide_partial_bytes(t, rows, u, sp);
       if (part > budget) continue;
       const int64_t wgs = mt * u * sp;
       const int64_t rounds = (wgs + 256 * t.per_cu - 1) / (256 * t.per_cu);
@@ -502,7 +502,7 @@ static size_t group_qmm_partials(const Group& g, int64_t rows) {
   const size_t least = group_qmm_partials_min(g, rows);
   if (!group_takes_wide(g, rows, group_partial_budget(g, rows), &sh)) return least;
   const WideTile& t = kWideTiles[sh.kind];
-  return std::max(least, wide_partial_bytes(t, sh.mtiles, group_units(g, 32 * t.nw), sh.splits));
+  return std::max(least, wide_partial_bytes(t, rows, group_units(g, 32 * t.nw), sh.splits));
 }
 
 // Scratch bytes (after the counter region) of one group launch.
@@ -647,6 +647,18 @@ static int run_group_qmv(const Group& g, const void* x, int x_type, int64_t rows
   return check_launch("EXL3 QMV launch");
 }
 
+// Whether a QMM's prologue (and the SwiGLU edge's, over the same rows and width)
+// takes the MFMA form, one wave per 16 rows x 128 inputs: once that puts two waves on
+// every SIMD.  Below, the form with 16 lanes per row and block spreads further.  Median
+// us of the lane form against the MFMA form, by waves of the latter: prologue 64
+// (17 x 4096) 3.2 / 4.6, 336 (47 x 14336) 4.2 / 4.6, 1024 (512 x 4096) 4.3 / 4.7, 2048
+// (1024 x 4096) 5.6 / 5.6, 3584 (512 x 14336) 9.0 / 8.1, 4096 9.8 / 8.7, 14336 (2048 x
+// 14336) 28.1 / 24.7; SwiGLU edge 896 4.8 / 5.5, 1024 5.0 / 5.6, 3584 12.9 / 12.6,
+// 14336 47 / 41.
+static bool qmm_mfma_prologue(int64_t rows, int in) {
+  return (rows + 15) / 16 * (in / 128) >= 2048;
+}
+
 // Prologue (one launch for all members) and one QMM over the group.
 // xhats: per member, null to run the prologue into the scratch.
 static int run_group_qmm(const Group& g, const void* x, int x_type, int64_t rows,
@@ -665,7 +677,10 @@ static int run_group_qmm(const Group& g, const void* x, int x_type, int64_t rows
       pp.suh[i] = g.parts[i]->suh;
       pp.xhat[i] = (uint16_t*)(scratch + i * xbytes);
     }
-    launch_prologue16(pp, g.count, stream);
+    if (qmm_mfma_prologue(rows, g.in))
+      launch_prologue16(pp, g.count, stream);
+    else
+      launch_prologue(pp, g.count, stream);
     if (int rc = check_launch("EXL3 prologue launch")) return rc;
   }
   int cblk0 = 0;
@@ -697,7 +712,7 @@ static int run_group_qmm(const Group& g, const void* x, int x_type, int64_t rows
     kWide[ws.kind][g.k - 1][g.cb](w, dim3((unsigned)wgs), stream);
     if (w.splits > 1) {
       if (int rc = check_launch("EXL3 QMM launch")) return rc;
-      launch_wide_reduce(w, t.r, t.nw, stream);
+      launch_wide_reduce(w, t.nw, stream);
     }
     return check_launch("EXL3 QMM launch");
   }
@@ -822,7 +837,7 @@ static int mlp_forward(const exl3_linear* gate, const exl3_linear* up, const exl
     return rc;
   if (int rc = launch_gate("SwiGLU prepare launch")) return rc;
   launch_swiglu_prepare((const uint16_t*)gu_y[0], (const uint16_t*)gu_y[1], down->suh, gate->out,
-                        (int)rows, act, stream);
+                        (int)rows, act, qmm_mfma_prologue(rows, gate->out), stream);
   if (int rc = check_launch("SwiGLU prepare launch")) return rc;
   return run_group_qmm(d, nullptr, EXL3_F16, rows, dy, counters, scratch, scratch_bytes, act,
                        stream);

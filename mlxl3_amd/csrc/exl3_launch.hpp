@@ -50,9 +50,9 @@ void launch_moe_route16(const MoePlanParams& pp, const MoeGatherParams& gp, size
 void launch_prologue(const PrologueParams& p, int members, hipStream_t s);
 // The same for the QMM (more than 16 rows): the Hadamard by MFMA.
 void launch_prologue16(const PrologueParams& p, int members, hipStream_t s);
-// Sums the split-K partials of a kWide launch of 16*R rows x 32*NW columns per
-// workgroup and finishes its outputs.
-void launch_wide_reduce(const WideParams& p, int R, int NW, hipStream_t s);
+// Sums the split-K partials of a kWide launch with 32*NW columns per workgroup and
+// finishes its outputs.
+void launch_wide_reduce(const WideParams& p, int NW, hipStream_t s);
 // values[i] = codeword(states[i], cb).
 void launch_codewords(const uint16_t* states, int64_t n, int cb, uint16_t* values, hipStream_t s);
 // packed[t][16k] = the trellis tile of states[t][256] (low k bits of each).
@@ -61,9 +61,10 @@ void launch_pack_tiles(const uint16_t* states, int64_t tiles, int k, uint16_t* p
 // y = f16(x . W) over decoded tiles (no glue).
 void launch_qmv_inner(const uint16_t* values, const uint16_t* x, int rows, int cols, uint16_t* y,
                       hipStream_t s);
-// xhat = the down projection's prologue of swiglu(gate, up), [rows][H].
+// xhat = the down projection's prologue of swiglu(gate, up), [rows][H]; `mfma`: with
+// the Hadamard as in launch_prologue16.
 void launch_swiglu_prepare(const uint16_t* gate, const uint16_t* up, const uint16_t* down_suh,
-                           int H, int rows, uint16_t* xhat, hipStream_t s);
+                           int H, int rows, uint16_t* xhat, bool mfma, hipStream_t s);
 // out[i] = swiglu(gate[i], up[i]) (Array::swiglu) or geglu(gate[i], up[i])
 // (Array::geglu) in f16.
 void launch_glu(const uint16_t* gate, const uint16_t* up, uint16_t* out, int64_t n, bool gelu,

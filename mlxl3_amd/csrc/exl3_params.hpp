@@ -70,7 +70,7 @@ struct WideMember {
 struct WideParams {
   WideMember mem[kMaxMembers];
   int members;
-  float* partials;     // [splits][tiles][16*R x 32*NW f32 in fragment order] (splits > 1)
+  float* partials;     // [splits][units][row blocks][16 x 32*NW f32 in fragment order]
   uint32_t* counters;  // [mtiles * pairs], zero between calls (splits > 1)
   int in, M, x_dtype;
   int units;   // column units of all members

@@ -15,6 +15,10 @@ template __global__ void prologue_kernel<true>(PrologueParams);
 template __global__ void prologue_kernel<false>(PrologueParams);
 template __global__ void prologue16_kernel<true>(PrologueParams);
 template __global__ void prologue16_kernel<false>(PrologueParams);
+template __global__ void swiglu_prepare16_kernel<true>(const uint16_t*, const uint16_t*,
+                                                       const uint16_t*, int, int, uint16_t*);
+template __global__ void swiglu_prepare16_kernel<false>(const uint16_t*, const uint16_t*,
+                                                        const uint16_t*, int, int, uint16_t*);
 template __global__ void swiglu_prepare_kernel<true>(const uint16_t*, const uint16_t*,
                                                      const uint16_t*, int, int, uint16_t*);
 template __global__ void swiglu_prepare_kernel<false>(const uint16_t*, const uint16_t*,
@@ -118,14 +122,13 @@ void launch_glu(const uint16_t* gate, const uint16_t* up, uint16_t* out, int64_t
 }
 
 void launch_swiglu_prepare(const uint16_t* gate, const uint16_t* up, const uint16_t* down_suh,
-                           int H, int rows, uint16_t* xhat, hipStream_t s) {
-  const unsigned groups = (unsigned)(((int64_t)((rows + 15) / 16) * (H / 128) + 3) / 4);
-  if ((((uintptr_t)gate | (uintptr_t)up | (uintptr_t)down_suh | (uintptr_t)xhat) & 15) == 0)
-    hipLaunchKernelGGL(swiglu_prepare_kernel<true>, dim3(groups), dim3(256), 0, s, gate, up,
-                       down_suh, H, rows, xhat);
-  else
-    hipLaunchKernelGGL(swiglu_prepare_kernel<false>, dim3(groups), dim3(256), 0, s, gate, up,
-                       down_suh, H, rows, xhat);
+                           int H, int rows, uint16_t* xhat, bool mfma, hipStream_t s) {
+  const bool vec = (((uintptr_t)gate | (uintptr_t)up | (uintptr_t)down_suh | (uintptr_t)xhat) & 15) == 0;
+  const unsigned groups = mfma ? (unsigned)(((int64_t)((rows + 15) / 16) * (H / 128) + 3) / 4)
+                               : (unsigned)(((int64_t)rows * (H / 128) + 15) / 16);
+  const auto kernel = mfma ? (vec ? swiglu_prepare16_kernel<true> : swiglu_prepare16_kernel<false>)
+                           : (vec ? swiglu_prepare_kernel<true> : swiglu_prepare_kernel<false>);
+  hipLaunchKernelGGL(kernel, dim3(groups), dim3(256), 0, s, gate, up, down_suh, H, rows, xhat);
 }
 
 void launch_fill_zero(uint32_t* p, size_t words, hipStream_t s) {

@@ -229,11 +229,44 @@ __global__ __launch_bounds__(256) void prologue16_kernel(PrologueParams p) {
 // xhat_down = f16(H128(f16(swiglu(g, u) * down_suh)) / sqrt(128)) (the down
 // projection's prologue applied to the activation, as the reference's
 // flash_up_finish_swiglu_prepare fuses them, exl3.metal:265-291, with
-// Array::swiglu's f16 arithmetic), the Hadamard as in prologue16_kernel.  grid
-// (ceil(ceil(rows / 16) * H / 128 / 4)), 256 threads.
+// Array::swiglu's f16 arithmetic).  16 lanes per (row, 128-block) job, 8
+// columns per lane (finish8).  grid (ceil(rows * H / 128 / 16)), 256 threads.
 template <bool VEC>
 __global__ __launch_bounds__(256) void swiglu_prepare_kernel(const uint16_t* __restrict__ gate,
                                                              const uint16_t* __restrict__ up,
+                                                             const uint16_t* __restrict__ down_suh,
+                                                             int H, int rows,
+                                                             uint16_t* __restrict__ xhat) {
+  int row, b;
+  const bool live = job16(rows, H >> 7, row, b);
+  const int c = b * 128 + 8 * (threadIdx.x & 15);
+  const size_t e = (size_t)row * H + c;
+  float a[8], sv[8];
+  if constexpr (VEC) {
+    const u32x4 gw = *(const u32x4*)(gate + e), uw = *(const u32x4*)(up + e);
+    const u32x4 sw = *(const u32x4*)(down_suh + c);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      a[2 * i] = swiglu_f16(h2f((uint16_t)gw[i]), h2f((uint16_t)uw[i]));
+      a[2 * i + 1] = swiglu_f16(h2f((uint16_t)(gw[i] >> 16)), h2f((uint16_t)(uw[i] >> 16)));
+      sv[2 * i] = h2f((uint16_t)sw[i]);
+      sv[2 * i + 1] = h2f((uint16_t)(sw[i] >> 16));
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      a[i] = swiglu_f16(h2f(gate[e + i]), h2f(up[e + i]));
+      sv[i] = h2f(down_suh[c + i]);
+    }
+  }
+  finish8<VEC>(a, sv, xhat + e, live, threadIdx.x & 63);
+}
+
+// The same for many rows, with the Hadamard as in prologue16_kernel.  grid
+// (ceil(ceil(rows / 16) * H / 128 / 4)), 256 threads.
+template <bool VEC>
+__global__ __launch_bounds__(256) void swiglu_prepare16_kernel(const uint16_t* __restrict__ gate,
+                                                               const uint16_t* __restrict__ up,
                                                              const uint16_t* __restrict__ down_suh,
                                                              int H, int rows,
                                                              uint16_t* __restrict__ xhat) {
@@ -497,7 +530,6 @@ __global__ __launch_bounds__(512) void qmm_kernel(QmmParams p) {
   const Member mm = select_member(p, cblk);
   const int cblk_l = cblk - mm.cblk0;  // column block inside the member
   const int TN = mm.out >> 4;
-  const int TO = p.total_out;
   const int nq_all = p.in >> 6;
   const int qa = split * nq_all / p.splits, nq = (split + 1) * nq_all / p.splits - qa;
   const int qlast = nq - 1;

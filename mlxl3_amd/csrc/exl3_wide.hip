@@ -21,9 +21,9 @@ template <int K, int CB>
 static void run_wide_8x8(const WideParams& p, dim3 g, hipStream_t s) { run_wide<K, CB, 8, 8>(p, g, s); }
 template <int K, int CB>
 static void run_wide_16x8(const WideParams& p, dim3 g, hipStream_t s) { run_wide<K, CB, 16, 8>(p, g, s); }
-void launch_wide_reduce(const WideParams& p, int R, int NW, hipStream_t s) {
-  const unsigned jobs = (unsigned)p.mtiles * p.units * R * (NW / 4);
-  hipLaunchKernelGGL(wide_reduce_kernel, dim3((jobs + 3) / 4), dim3(256), 0, s, p, R, NW);
+void launch_wide_reduce(const WideParams& p, int NW, hipStream_t s) {
+  const unsigned jobs = (unsigned)p.units * ((p.M + 15) / 16) * (NW / 4);
+  hipLaunchKernelGGL(wide_reduce_kernel, dim3((jobs + 3) / 4), dim3(256), 0, s, p, NW);
 }
 const WideFn kWide[3][8][3] = {EXL3_TABLE(run_wide_4x4), EXL3_TABLE(run_wide_8x8),
                                EXL3_TABLE(run_wide_16x8)};

@@ -502,14 +502,17 @@ __global__ __launch_bounds__(64 * NW) void wide_qmm_kernel(WideParams p) {
   wide_mm<K, CB, R, NW, false>(lds, asrc, wsrc, aoff, woff, nq, R, wave, lane, acc);
 
   if (p.splits > 1) {
-    // split-K: the f32 sums, [split][tile][rb][wave][cg][lane] of 16 bytes, for
-    // wide_reduce_kernel
-    float* slab = p.partials + ((size_t)split * per_split + tile) * (C::kRows * C::kCols);
+    // split-K: the f32 sums, [split][unit][row block][wave][cg][lane] of 16 bytes,
+    // for wide_reduce_kernel (row blocks past M are left out)
+    const int blocks = (p.M + 15) >> 4;
+    float* dst = p.partials + ((size_t)split * p.units + unit) * blocks * (16 * C::kCols) +
+                 (size_t)mtile * R * (16 * C::kCols) + wave * 512 + lane * 4;
 #pragma unroll
     for (int rb = 0; rb < R; ++rb)
+      if (mtile * R + rb < blocks)
 #pragma unroll
-      for (int cg = 0; cg < 2; ++cg)
-        *(float4v*)(slab + ((rb * NW + wave) * 2 + cg) * 256 + lane * 4) = acc[rb][cg];
+        for (int cg = 0; cg < 2; ++cg)
+          *(float4v*)(dst + rb * (16 * C::kCols) + cg * 256) = acc[rb][cg];
     return;
   }
   uint16_t* ys = (uint16_t*)lds;
@@ -531,19 +534,16 @@ __global__ __launch_bounds__(64 * NW) void wide_qmm_kernel(WideParams p) {
 // columns adds the parts in split order.  A launch of its own: every CU takes
 // part and the partials go through the caches, where the last arriver of a tile
 // summing them alone (coherent loads, one workgroup per tile) was the larger
-// half of such calls.  grid ceil(mtiles * R * units * NW / 4 / 4), 256 threads.
-static __global__ __launch_bounds__(256) void wide_reduce_kernel(WideParams p, int R, int NW) {
+// half of such calls.  grid ceil(units * ceil(M / 16) * NW / 4 / 4), 256 threads.
+static __global__ __launch_bounds__(256) void wide_reduce_kernel(WideParams p, int NW) {
   __shared__ __attribute__((aligned(16))) uint16_t ys[4][16 * kYStride];
   __shared__ __attribute__((aligned(16))) uint16_t s_svh[4][128], s_bias[4][128];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int tiles = p.mtiles * p.units;
-  const int kh = NW / 4, job = blockIdx.x * 4 + wave;
-  const int half = job % kh, tr = job / kh;  // tr = tile * R + row block
-  const int tile = tr / R, rb = tr - tile * R;
-  const int mtile = tile / p.units, unit = tile - mtile * p.units;
-  const int row0 = (mtile * R + rb) * 16;
-  if (tile >= tiles || row0 >= p.M) return;  // uniform per wave
+  const int kh = NW / 4, blocks = (p.M + 15) >> 4, job = blockIdx.x * 4 + wave;
+  const int half = job % kh, ub = job / kh;  // ub = unit * blocks + row block
+  const int unit = ub / blocks, row0 = (ub - unit * blocks) * 16;
+  if (unit >= p.units) return;  // uniform per wave
   const WideMember mm = select_wide(p, unit);
   const int col0 = (unit - mm.unit0) * 32 * NW + 128 * half;
   if (col0 >= mm.out) return;
@@ -552,8 +552,8 @@ static __global__ __launch_bounds__(256) void wide_reduce_kernel(WideParams p, i
     s_svh[wave][i] = mm.svh[col0 + i];
     s_bias[wave][i] = mm.bias ? mm.bias[col0 + i] : 0;
   }
-  const size_t slab = (size_t)R * 16 * 32 * NW, sstride = (size_t)tiles * slab;
-  const float* src = p.partials + (size_t)tile * slab + (rb * NW + 4 * half) * 512 + lane * 4;
+  const size_t sstride = (size_t)p.units * blocks * 512 * NW;
+  const float* src = p.partials + ((size_t)ub * NW + 4 * half) * 512 + lane * 4;
   float4v sum[8];
 #pragma unroll
   for (int f = 0; f < 8; ++f) sum[f] = *(const float4v*)(src + f * 256);

@@ -114,6 +114,54 @@ def test_workspace_between_the_two_needs(monkeypatch):
 
 
 # ---------------------------------------------------------------------------
+# the input prologue and the SwiGLU edge by MFMA (from 2048 waves of 16 x 128 on)
+# ---------------------------------------------------------------------------
+@pytest.mark.parametrize("rows", [2032, 2033, 2048])
+@pytest.mark.parametrize("dtype", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("off", [0, 1])
+def test_prologue_on_both_sides_of_the_rule(rows, dtype, off):
+    """2032 rows x 2048 inputs are 127 * 16 waves (16 lanes per row), 2033 and 2048
+    are 128 * 16 (MFMA), the first with one row in its last block; `off`: an input one
+    element past its alignment (the scalar loads)."""
+    import torch
+
+    print(f"prologue rows={rows} {dtype} off={off}", flush=True)
+    lin, (tr, suh, svh, _) = make_layer(8000, 2048, 128, 4, 0)
+    x = synth.activations(9, 1, rows, 2048)
+    t = torch.from_numpy(x).cuda().to({"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}[dtype])
+    buf = torch.empty(rows * 2048 + off, dtype=t.dtype, device="cuda")
+    t = buf[off:].view(rows, 2048).copy_(t)
+    pick = np.array([0, 1, 15, 16, 1000, rows - 2, rows - 1])
+    y = lin.forward(t).float().cpu().numpy().astype(np.float64)[pick]
+    want = oracle.forward(t[pick].half().cpu().numpy(), tr, suh, svh, 4, 0, mode=1).astype(np.float64)
+    if dtype == "bf16":
+        want = (bf16_bits(want).astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    # 2 ulp of the f16 result, one more of the last rounded format
+    assert np.abs(y - want).max() <= 3 * ulp_of(np.abs(want).max(), dtype == "bf16")
+
+
+@pytest.mark.parametrize("rows", [2032, 2033])
+@pytest.mark.parametrize("off", [0, 1])
+def test_swiglu_edge_on_both_sides_of_the_rule(rows, off):
+    """The edge of 2048 hidden columns: the fused MLP against its own parts, with the
+    down projection's input scales aligned and not, and against the oracle."""
+    import mlxl3_amd
+    import torch
+    import test_gpu_group as g
+
+    print(f"swiglu edge rows={rows} off={off}", flush=True)
+    _, (gate, up, down), host = g.mlp_case(256, 2048, 3, 1)
+    suh = torch.empty(2048 + off, dtype=torch.float16, device="cuda")[off:].copy_(down.suh)
+    down = mlxl3_amd.Exl3Linear(down.trellis, suh, down.svh, None, 3, 1)
+    x_np = synth.activations(10, 1, rows, 256)
+    x = torch.from_numpy(x_np).cuda()
+    y, other = mlxl3_amd.Exl3Mlp(gate, up, down).forward(x), g.unfused((gate, up, down), x)
+    assert torch.equal(y.view(torch.int16), other.view(torch.int16))
+    pick = [0, 17, rows - 1]
+    g.check_tol(y.cpu().numpy()[pick], oracle.mlp_forward(x_np[pick], *host), "rows of the oracle")
+
+
+# ---------------------------------------------------------------------------
 # the expert QMMs for many rows per expert
 # ---------------------------------------------------------------------------
 @pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 6, 8])
