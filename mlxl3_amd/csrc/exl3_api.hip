@@ -470,6 +470,11 @@ static int group_units(const Group& g, int cols) {
 // producer/consumer kernel (whose model leaves out ~6 us of ring fill and
 // epilogue).  Its trellis copies are 16 bytes wide, so every trellis has to be
 // 16-byte aligned (a checkpoint's tensors are; a caller's view may not be).
+// Two corrections: with splits its sums take a launch more, which a call of less than
+// ~25 us (20 in the model) cannot hide from the host (us a call, producer/consumer
+// kernel against this one: 32 rows x 4096 x 3968 19.3 / 22.7, 71 x 2048 x 1536 18.6 /
+// 21.5, 36 x 4096 x 5888 21.2 / 23.0); and two MB = 1 workgroups share a CU, which the
+// model leaves out past 256 of them (18 x 22656 x 22656 142 / 152 to 170).
 // EXL3_WIDE=0/1 forces it off or on (tuning).
 static bool group_takes_wide(const Group& g, int64_t rows, size_t budget, WideShape* shape) {
   for (int i = 0; i < g.count; ++i)
@@ -477,7 +482,10 @@ static bool group_takes_wide(const Group& g, int64_t rows, size_t budget, WideSh
   const int units[2] = {group_units(g, 128), group_units(g, 256)};
   *shape = choose_wide_shape(g.in, units, rows, budget);
   if (const char* env = getenv("EXL3_WIDE")) return atoi(env) != 0;
-  return shape->cost < choose_qmm_shape(g.in, g.total_out, rows).cost + 6000.0;
+  const QmmShape q = choose_qmm_shape(g.in, g.total_out, rows);
+  if (shape->splits > 1 && q.cost < 20000.0) return false;
+  const int64_t wgs = (int64_t)q.mtiles * (g.total_out / 128) * q.splits;
+  return shape->cost < (q.mb == 1 && wgs > 256 ? 0.75 : 1.0) * q.cost + 6000.0;
 }
 
 // Split-K partials of the producer/consumer QMM over the group: what every

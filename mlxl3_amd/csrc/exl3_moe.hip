@@ -99,7 +99,10 @@ int moe_splits(const exl3_moe* h, int64_t slots, int block_rows, int k_in, int c
 // new; rows per expert): 128 experts top-8 K = 3, 2048x768: 62 264 -> 298, 125 451 ->
 // 376, 250 825 -> 739; 64 experts top-6 K = 4, 2048x1024: 56 168 -> 188, 188 406 -> 425;
 // 8 experts top-2: 64 80 -> 87, 250 132 -> 106, 1000 268 -> 242; 32 experts top-4 K = 5,
-// 3072x1536: 125 362 -> 264.  Its copies address the bank and the gathered rows with
+// 3072x1536: 125 362 -> 264.  Not where the last round of two workgroups per CU would be
+// mostly empty (8 experts, 687 rows each: 1.25 rounds, 195 -> 202), and for GELU, whose
+// glue in a launch of its own costs more (its binary64 tanh), only above 112 rows per
+// expert (70 364 -> 384, 113 487 -> 479, 125 524 -> 500).  Its copies address the bank and the gathered rows with
 // 32-bit byte offsets, 16 bytes at a time.  Pinned split counts or block rows keep
 // moe_mm_kernel.  EXL3_MOE_WIDE=0/1 forces it off or on (tuning).
 bool moe_takes_wide(const exl3_moe* h, int64_t slots) {
@@ -113,7 +116,12 @@ bool moe_takes_wide(const exl3_moe* h, int64_t slots) {
   if (h->force_splits > 1 || getenv("EXL3_MOE_BLOCK_ROWS")) return false;
   if (const char* env = getenv("EXL3_MOE_WIDE")) return atoi(env) != 0;
   const int64_t avg = slots / h->experts, rows_wide = moe_wide_rows(h->k);
-  return avg > 64 && (avg + 63) / 64 >= 2 * ((avg + rows_wide - 1) / rows_wide);
+  if (avg <= (h->gelu ? 112 : 64)) return false;
+  const int64_t blocks = (avg + rows_wide - 1) / rows_wide;
+  if ((avg + 63) / 64 < 2 * blocks) return false;
+  const int64_t wgs = h->experts * blocks * (2 * h->hidden / 128), slots_cu = 512;  // two per CU
+  const int64_t rounds = (wgs + slots_cu - 1) / slots_cu;
+  return rounds == 1 || 4 * wgs >= 3 * rounds * slots_cu;
 }
 
 // The small-row path (decode): up to this many routed slots run as two
