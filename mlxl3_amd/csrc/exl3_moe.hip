@@ -103,7 +103,8 @@ int moe_splits(const exl3_moe* h, int64_t slots, int block_rows, int k_in, int c
 // mostly empty (8 experts, 687 rows each: 1.25 rounds, 195 -> 202), and for GELU, whose
 // glue in a launch of its own costs more (its binary64 tanh), only above 112 rows per
 // expert (70 364 -> 384, 113 487 -> 479, 125 524 -> 500).  Its copies address the bank and the gathered rows with
-// 32-bit byte offsets, 16 bytes at a time.  Pinned split counts or block rows keep
+// 32-bit byte offsets, 16 bytes at a time.  Pinned split counts (one split among them:
+// a row of such a bank has the same bits in every call) or block rows keep
 // moe_mm_kernel.  EXL3_MOE_WIDE=0/1 forces it off or on (tuning).
 bool moe_takes_wide(const exl3_moe* h, int64_t slots) {
   const int64_t bank = std::max((int64_t)2 * h->experts * h->hidden / 8 * h->k * h->in,
@@ -113,7 +114,7 @@ bool moe_takes_wide(const exl3_moe* h, int64_t slots) {
   if (((uintptr_t)h->gu_trellis | (uintptr_t)h->down_trellis) & 15) return false;
   // the gate's and up's sums borrow the slot outputs' buffer (f32 rows of `in`)
   if (h->hidden > h->in || h->hidden / 128 > 65535) return false;
-  if (h->force_splits > 1 || getenv("EXL3_MOE_BLOCK_ROWS")) return false;
+  if (h->force_splits > 0 || getenv("EXL3_MOE_BLOCK_ROWS")) return false;
   if (const char* env = getenv("EXL3_MOE_WIDE")) return atoi(env) != 0;
   const int64_t avg = slots / h->experts, rows_wide = moe_wide_rows(h->k);
   if (avg <= (h->gelu ? 112 : 64)) return false;

@@ -122,6 +122,23 @@ def test_moe_rows_independent_and_deterministic(monkeypatch):
           "moe single row, default splits")
 
 
+@pytest.mark.parametrize("activation", ["silu", "gelu"])
+def test_moe_pinned_single_split_rows_independent_at_prefill_size(activation, monkeypatch):
+    """One split pinned: a row of a call that gives every expert 160 rows (where
+    unpinned banks may take the QMMs in registers) equals the row run alone, for a
+    sample of rows, and the call equals itself with those QMMs forced off."""
+    print(f"moe pinned single split, 160 rows per expert, {activation}", flush=True)
+    monkeypatch.setenv("EXL3_MOE_SPLITS", "1")
+    layer, x, sel, sc = case(1792, 768, 4, 2, 320, 4, 131)  # 28 steps: one split alone too
+    x = synth.activations(131, 510, 320, 1792, outlier_frac=0.01)
+    moe = make_moe(layer, 2, 4, 0, activation=activation)
+    y = run(moe, x, sel, sc)
+    for r in range(0, 320, 8):
+        np.testing.assert_array_equal(run(moe, x[r:r + 1], sel[r:r + 1], sc[r:r + 1]), y[r:r + 1])
+    monkeypatch.setenv("EXL3_MOE_WIDE", "0")
+    np.testing.assert_array_equal(run(moe, x, sel, sc), y)
+
+
 @pytest.mark.parametrize("splits", [1, 3, 8])
 def test_moe_split_k_schedules(splits, monkeypatch):
     print(f"moe splits={splits}", flush=True)
