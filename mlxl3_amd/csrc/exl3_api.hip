@@ -279,14 +279,21 @@ struct QmmShape {
   double cost;  // modelled ns
 };
 
-static QmmShape choose_qmm_shape(int in, int out, int64_t rows) {
-  const int col_blocks = out / 128, nq = in / 64;
-  int force_mb = 0, force_splits = 0;
-  if (const char* env = getenv("EXL3_QMM_MB")) {
-    int v = atoi(env);
-    if (v == 1 || v == 2 || v == 4) force_mb = v;
+// EXL3_QMM_MB and EXL3_QMM_SPLITS (0: not pinned).
+struct QmmPins {
+  int mb = 0, splits = 0;
+  QmmPins() {
+    if (const char* env = getenv("EXL3_QMM_MB")) {
+      int v = atoi(env);
+      if (v == 1 || v == 2 || v == 4) mb = v;
+    }
+    if (const char* env = getenv("EXL3_QMM_SPLITS")) splits = std::max(0, atoi(env));
   }
-  if (const char* env = getenv("EXL3_QMM_SPLITS")) force_splits = std::max(0, atoi(env));
+};
+
+static QmmShape choose_qmm_shape(int in, int out, int64_t rows, const QmmPins& pins = QmmPins()) {
+  const int col_blocks = out / 128, nq = in / 64;
+  const int force_mb = pins.mb, force_splits = pins.splits;
   QmmShape best{4, (int)((rows + 255) / 256), 1, 0};
   double best_cost = 1e300;
   for (int mb : {4, 2, 1}) {
@@ -475,14 +482,17 @@ static int group_units(const Group& g, int cols) {
 // kernel against this one: 32 rows x 4096 x 3968 19.3 / 22.7, 71 x 2048 x 1536 18.6 /
 // 21.5, 36 x 4096 x 5888 21.2 / 23.0); and two MB = 1 workgroups share a CU, which the
 // model leaves out past 256 of them (18 x 22656 x 22656 142 / 152 to 170).
-// EXL3_WIDE=0/1 forces it off or on (tuning).
+// EXL3_WIDE=0/1 forces it off or on (tuning); without it, a pinned shape of the
+// producer/consumer kernel keeps that kernel.
 static bool group_takes_wide(const Group& g, int64_t rows, size_t budget, WideShape* shape) {
   for (int i = 0; i < g.count; ++i)
     if ((uintptr_t)g.parts[i]->trellis & 15) return false;
   const int units[2] = {group_units(g, 128), group_units(g, 256)};
   *shape = choose_wide_shape(g.in, units, rows, budget);
   if (const char* env = getenv("EXL3_WIDE")) return atoi(env) != 0;
-  const QmmShape q = choose_qmm_shape(g.in, g.total_out, rows);
+  const QmmPins pins;
+  if (pins.mb || pins.splits) return false;
+  const QmmShape q = choose_qmm_shape(g.in, g.total_out, rows, pins);
   if (shape->splits > 1 && q.cost < 20000.0) return false;
   const int64_t wgs = (int64_t)q.mtiles * (g.total_out / 128) * q.splits;
   return shape->cost < (q.mb == 1 && wgs > 256 ? 0.75 : 1.0) * q.cost + 6000.0;

@@ -48,5 +48,5 @@ def test_pinned_qmm_shape_keeps_its_kernel(monkeypatch, linear, env, n_in, n_out
     # EXL3_WIDE=1 still forces the QMM in registers
     monkeypatch.setenv("EXL3_WIDE", "1")
     monkeypatch.setenv("EXL3_WIDE_TILE", "1")
-    monkeypatch.setenv("EXL3_WIDE_SPLITS", "8")
-    assert need(rows) >= xhat_bytes(rows, n_in) + 4 * 8 * rows * n_out
+    monkeypatch.setenv("EXL3_WIDE_SPLITS", "2")
+    assert need(rows) >= xhat_bytes(rows, n_in) + 4 * 2 * rows * n_out
