@@ -20,8 +20,8 @@ struct MoeMmParams;
 struct MoePlanParams;
 struct MoeGatherParams;
 // (parameters, gate/up with the GLU edge or down, blocks rounded up to 8, the
-// edge's [2][slots][hidden] f16 scratch, stream)
-typedef void (*MoeWideFn)(const MoeMmParams&, bool, int, uint16_t*, hipStream_t);
+// edge's [2][slots][hidden] f16 scratch, stream); EXL3_OK or the failed launch's code
+typedef int (*MoeWideFn)(const MoeMmParams&, bool, int, uint16_t*, hipStream_t);
 typedef void (*DecodeFn)(const uint32_t*, int64_t, uint16_t*, uint16_t*, dim3, hipStream_t);
 
 // Every workspace starts with this many bytes of counters that are zero

@@ -481,16 +481,16 @@ int exl3_moe_forward(const exl3_moe* h, const void* x, int32_t x_type, int64_t r
   d.scores = scores;
   d.scores_dtype = scores_type;
   d.z = ws + L.z;
-  if (L.wide)
-    kMoeWide[h->k - 1][h->cb](q, true, grid_blocks, (uint16_t*)d.z, s);
-  else
+  if (L.wide) {
+    const MoeWideFn wide = kMoeWide[h->k - 1][h->cb];
+    if (int rc = wide(q, true, grid_blocks, (uint16_t*)d.z, s)) return rc;
+    if (int rc = wide(d, false, grid_blocks, nullptr, s)) return rc;
+  } else {
     gateup<<<grid_blocks * q.col_blocks * q.splits, 512, 0, s>>>(q);
-  if (int rc = check_launch("moe gate/up")) return rc;
-  if (L.wide)
-    kMoeWide[h->k - 1][h->cb](d, false, grid_blocks, nullptr, s);
-  else
+    if (int rc = check_launch("moe gate/up")) return rc;
     down<<<grid_blocks * d.col_blocks * d.splits, 256, 0, s>>>(d);
-  if (int rc = check_launch("moe down")) return rc;
+    if (int rc = check_launch("moe down")) return rc;
+  }
 
   const dim3 rgrid((unsigned)rows, (h->in + 2047) / 2048);
   if (((uintptr_t)y & 15) == 0)

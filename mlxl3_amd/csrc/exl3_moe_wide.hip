@@ -34,22 +34,25 @@ void launch_moe_route16(const MoePlanParams& pp, const MoeGatherParams& gp, size
 }
 
 template <int K, int CB>
-static void run_moe_wide(const MoeMmParams& p, bool gate_up, int blocks, uint16_t* raw,
-                         hipStream_t s) {
+static int run_moe_wide(const MoeMmParams& p, bool gate_up, int blocks, uint16_t* raw,
+                        hipStream_t s) {
   if (!gate_up) {
     const int units = p.width / 128;
     hipLaunchKernelGGL((moe_wide_kernel<K, CB, 1>), dim3((unsigned)blocks * units), dim3(256), 0, s,
                        p, units, raw);
-    return;
+    return check_launch("moe down");
   }
   const int units = 2 * (p.width / 128);
   hipLaunchKernelGGL((moe_wide_kernel<K, CB, 2>), dim3((unsigned)blocks * units), dim3(256), 0, s, p,
                      units, raw);
+  if (int rc = check_launch("moe gate/up")) return rc;
+  if (int rc = launch_gate("moe glu")) return rc;
   const dim3 grid((unsigned)blocks, p.width / 128);
   if (p.gelu)
     hipLaunchKernelGGL(moe_glu_kernel<true>, grid, dim3(256), 0, s, p, raw);
   else
     hipLaunchKernelGGL(moe_glu_kernel<false>, grid, dim3(256), 0, s, p, raw);
+  return check_launch("moe glu");
 }
 #define EXL3_MOE_WIDE_ROW(K) {run_moe_wide<K, 0>, run_moe_wide<K, 1>, run_moe_wide<K, 2>}
 const MoeWideFn kMoeWide[8][3] = {

@@ -66,6 +66,30 @@ def test_moe_failure_after_gate_up_keeps_output_and_workspace():
     assert torch.equal(y.view(torch.int16), y2.view(torch.int16))
 
 
+def test_moe_glu_launch_is_checked(monkeypatch):
+    """Where the gate/up glue is a launch of its own, its failure is reported under
+    its own name and nothing is launched after it."""
+    torch = torch_mod()
+    print("fault hook: moe glu", flush=True)
+    monkeypatch.setenv("EXL3_MOE_WIDE", "1")
+    in_f, hidden, E, top_k, k, rows = 256, 256, 2, 2, 3, 100
+    layer = synth.moe_layer(9, 110, in_f, hidden, E, k)
+    moe = mlxl3_amd.Exl3SwitchGlu(*[dev(a) for a in layer], top_k=top_k, k=k, cb=0)
+    x = dev(synth.activations(9, 1, rows, in_f))
+    sel, sc = synth.moe_routes(9, 2, rows, E, top_k)
+    sel, sc = dev(sel), dev(sc)
+    want = moe.forward(x, sel, sc)
+    mlxl3_amd.debug_fail_launch("moe glu")
+    try:
+        with pytest.raises(mlxl3_amd.Exl3Error, match="moe glu: forced launch failure"):
+            moe.forward(x, sel, sc)
+    finally:
+        mlxl3_amd.debug_fail_launch(None)
+    y = moe.forward(x, sel, sc)
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+
+
 def test_qmm_failure_after_prologue_keeps_output_and_workspace():
     torch = torch_mod()
     print("fault hook: QMM prologue", flush=True)
