@@ -472,81 +472,97 @@ static int group_units(const Group& g, int cols) {
   return units;
 }
 
-// Whether a QMM over the group runs in registers (exl3_wide.hpp) and in which
-// shape, with `budget` bytes for partials: where it is modelled faster than the
-// producer/consumer kernel (whose model leaves out ~6 us of ring fill and
-// epilogue).  Its trellis copies are 16 bytes wide, so every trellis has to be
-// 16-byte aligned (a checkpoint's tensors are; a caller's view may not be).
-// Two corrections: with splits its sums take a launch more, which a call of less than
-// ~25 us (20 in the model) cannot hide from the host (us a call, producer/consumer
-// kernel against this one: 32 rows x 4096 x 3968 19.3 / 22.7, 71 x 2048 x 1536 18.6 /
-// 21.5, 36 x 4096 x 5888 21.2 / 23.0); and two MB = 1 workgroups share a CU, which the
-// model leaves out past 256 of them (18 x 22656 x 22656 142 / 152 to 170).
-// EXL3_WIDE=0/1 forces it off or on (tuning); without it, a pinned shape of the
-// producer/consumer kernel keeps that kernel.
-static bool group_takes_wide(const Group& g, int64_t rows, size_t budget, WideShape* shape) {
-  for (int i = 0; i < g.count; ++i)
-    if ((uintptr_t)g.parts[i]->trellis & 15) return false;
+// What a QMM over the group runs (rows > 16).
+struct QmmPlan {
+  QmmShape q;       // the producer/consumer kernel's shape
+  WideShape w;      // the shape in registers (exl3_wide.hpp), if that may run
+  bool may_wide, forced_wide, wide;  // wide: it does
+  size_t least;     // bytes of partials that every workspace has to hold
+  size_t partials;  // ... and that the launch takes when it is given
+};
+
+static size_t wide_partials(const Group& g, int64_t rows, const WideShape& w) {
+  const WideTile& t = kWideTiles[w.kind];
+  return wide_partial_bytes(t, rows, group_units(g, 32 * t.nw), w.splits);
+}
+
+// Sets p.w to the fastest shape whose partials fit in `budget` bytes and p.wide to
+// whether it runs: where it is modelled faster than the producer/consumer kernel
+// (whose model leaves out ~6 us of ring fill and epilogue).  Two corrections: with
+// splits its sums take a launch more, which a call of less than ~25 us (20 in the
+// model) cannot hide from the host (us a call, producer/consumer kernel against this
+// one: 32 rows x 4096 x 3968 19.3 / 22.7, 71 x 2048 x 1536 18.6 / 21.5, 36 x 4096 x
+// 5888 21.2 / 23.0); and two MB = 1 workgroups share a CU, which the model leaves out
+// past 256 of them (18 x 22656 x 22656 142 / 152 to 170).
+static void plan_wide(const Group& g, int64_t rows, size_t budget, QmmPlan& p) {
   const int units[2] = {group_units(g, 128), group_units(g, 256)};
-  *shape = choose_wide_shape(g.in, units, rows, budget);
-  if (const char* env = getenv("EXL3_WIDE")) return atoi(env) != 0;
+  p.w = choose_wide_shape(g.in, units, rows, budget);
+  const int64_t wgs = (int64_t)p.q.mtiles * (g.total_out / 128) * p.q.splits;
+  p.wide = p.forced_wide ||
+           ((p.w.splits == 1 || p.q.cost >= 20000.0) &&
+            p.w.cost < (p.q.mb == 1 && wgs > 256 ? 0.75 : 1.0) * p.q.cost + 6000.0);
+}
+
+// The plan of a call, derived once per entry point.  The copies of the kernel in
+// registers are 16 bytes wide, so every trellis has to be 16-byte aligned (a
+// checkpoint's tensors are; a caller's view may not be).  EXL3_WIDE=0/1 forces it
+// off or on (tuning); without it, a pinned shape of the producer/consumer kernel
+// keeps that kernel.
+// Its partials may take any amount, but where the allocation-free entry point serves
+// the call (one projection that fits its fixed workspace at the least), no more
+// than fits there, so both entry points run the same shape and give the same bits.
+static QmmPlan plan_qmm(const Group& g, int64_t rows) {
   const QmmPins pins;
-  if (pins.mb || pins.splits) return false;
-  const QmmShape q = choose_qmm_shape(g.in, g.total_out, rows, pins);
-  if (shape->splits > 1 && q.cost < 20000.0) return false;
-  const int64_t wgs = (int64_t)q.mtiles * (g.total_out / 128) * q.splits;
-  return shape->cost < (q.mb == 1 && wgs > 256 ? 0.75 : 1.0) * q.cost + 6000.0;
-}
-
-// Split-K partials of the producer/consumer QMM over the group: what every
-// workspace has to hold.
-static size_t group_qmm_partials_min(const Group& g, int64_t rows) {
-  return qmm_partial_bytes(choose_qmm_shape(g.in, g.total_out, rows), g.total_out);
-}
-// The partials a launch may choose: any amount, but where the allocation-free
-// entry point serves the call (one projection that fits its fixed workspace at
-// the least), no more than fits there, so both entry points run the same shape
-// and give the same bits.
-static size_t group_partial_budget(const Group& g, int64_t rows) {
-  if (g.count > 1) return SIZE_MAX;
-  const size_t room = kNoAllocBytes - kWorkspaceCounterBytes;
-  const size_t xhat = align_up(sizeof(uint16_t) * (size_t)rows * g.in);
-  return xhat + align_up(group_qmm_partials_min(g, rows)) > room ? SIZE_MAX : room - xhat;
-}
-// ... and what the launch takes when it is given: a workspace between the two
-// gets the fastest shape that fits.
-static size_t group_qmm_partials(const Group& g, int64_t rows) {
-  WideShape sh;
-  const size_t least = group_qmm_partials_min(g, rows);
-  if (!group_takes_wide(g, rows, group_partial_budget(g, rows), &sh)) return least;
-  const WideTile& t = kWideTiles[sh.kind];
-  return std::max(least, wide_partial_bytes(t, rows, group_units(g, 32 * t.nw), sh.splits));
-}
-
-// Scratch bytes (after the counter region) of one group launch.
-static size_t group_scratch_bytes(const Group& g, int64_t rows) {
-  if (rows <= kQmvMaxRows) {
-    int splits, kw;
-    group_qmv_shape(g, &splits, &kw);
-    const size_t xhat = qmv_separate_prologue(g, rows, splits)
-                            ? g.count * align_up(sizeof(uint16_t) * (size_t)rows * g.in)
-                            : 0;
-    // partials: 8 KB fragment slabs per split and column block, or one
-    // row-major f32 row per split and row
-    const size_t partials = qmv_fragment_exchange(rows, kw)
-                                ? (size_t)splits * (g.total_out / 128) * 8192
-                                : sizeof(float) * (size_t)splits * rows * g.total_out;
-    return xhat + align_up(partials);
+  QmmPlan p{};
+  p.q = choose_qmm_shape(g.in, g.total_out, rows, pins);
+  p.least = p.partials = qmm_partial_bytes(p.q, g.total_out);
+  const char* env = getenv("EXL3_WIDE");
+  p.forced_wide = env && atoi(env) != 0;
+  p.may_wide = env ? p.forced_wide : !pins.mb && !pins.splits;
+  for (int i = 0; i < g.count; ++i)
+    if ((uintptr_t)g.parts[i]->trellis & 15) p.may_wide = false;
+  if (!p.may_wide) return p;
+  size_t budget = SIZE_MAX;
+  if (g.count == 1) {
+    const size_t room = kNoAllocBytes - kWorkspaceCounterBytes;
+    const size_t xhat = align_up(sizeof(uint16_t) * (size_t)rows * g.in);
+    if (xhat + align_up(p.least) <= room) budget = room - xhat;
   }
-  return (size_t)g.count * align_up(sizeof(uint16_t) * (size_t)rows * g.in) +
-         align_up(group_qmm_partials(g, rows));
+  plan_wide(g, rows, budget, p);
+  if (p.wide) p.partials = std::max(p.least, wide_partials(g, rows, p.w));
+  return p;
 }
 
-// ... that a call cannot do without.
-static size_t group_scratch_min(const Group& g, int64_t rows) {
-  if (rows <= kQmvMaxRows) return group_scratch_bytes(g, rows);
-  return (size_t)g.count * align_up(sizeof(uint16_t) * (size_t)rows * g.in) +
-         align_up(group_qmm_partials_min(g, rows));
+// The plan for a workspace with `room` bytes for partials: one between the two needs
+// gets the fastest shape that fits.
+static void fit_plan(const Group& g, int64_t rows, size_t room, QmmPlan& p) {
+  if (p.wide && wide_partials(g, rows, p.w) > room) plan_wide(g, rows, room, p);
+}
+
+// Scratch bytes of a QMM with `partials` bytes of partials.
+static size_t qmm_scratch(const Group& g, int64_t rows, size_t partials) {
+  return (size_t)g.count * align_up(sizeof(uint16_t) * (size_t)rows * g.in) + align_up(partials);
+}
+
+// Scratch bytes of a QMV (rows <= 16).
+static size_t qmv_scratch(const Group& g, int64_t rows) {
+  int splits, kw;
+  group_qmv_shape(g, &splits, &kw);
+  const size_t xhat = qmv_separate_prologue(g, rows, splits)
+                          ? g.count * align_up(sizeof(uint16_t) * (size_t)rows * g.in)
+                          : 0;
+  // partials: 8 KB fragment slabs per split and column block, or one
+  // row-major f32 row per split and row
+  const size_t partials = qmv_fragment_exchange(rows, kw)
+                              ? (size_t)splits * (g.total_out / 128) * 8192
+                              : sizeof(float) * (size_t)splits * rows * g.total_out;
+  return xhat + align_up(partials);
+}
+
+// Scratch bytes (after the counter region) that one group launch makes use of.
+static size_t group_scratch_bytes(const Group& g, int64_t rows) {
+  if (rows <= kQmvMaxRows) return qmv_scratch(g, rows);
+  return qmm_scratch(g, rows, plan_qmm(g, rows).partials);
 }
 
 static int check_rows(const Group& g, int64_t rows) {
@@ -679,7 +695,7 @@ static bool qmm_mfma_prologue(int64_t rows, int in) {
 
 // Prologue (one launch for all members) and one QMM over the group.
 // xhats: per member, null to run the prologue into the scratch.
-static int run_group_qmm(const Group& g, const void* x, int x_type, int64_t rows,
+static int run_group_qmm(const Group& g, QmmPlan plan, const void* x, int x_type, int64_t rows,
                          void* const* ys, uint32_t* counters, char* scratch, size_t scratch_bytes,
                          const uint16_t* given_xhat, hipStream_t stream) {
   if (int rc = launch_gate("EXL3 QMM launch")) return rc;
@@ -708,9 +724,9 @@ static int run_group_qmm(const Group& g, const void* x, int x_type, int64_t rows
     cblk0 += g.parts[i]->out / 128;
   }
   const size_t xhats = given_xhat ? 0 : g.count * xbytes;
-  WideShape ws;
-  if (group_takes_wide(g, rows, std::min(group_partial_budget(g, rows), scratch_bytes - xhats),
-                       &ws) && ((uintptr_t)q.mem[0].xhat & 15) == 0) {
+  fit_plan(g, rows, scratch_bytes - xhats, plan);
+  if (plan.wide && ((uintptr_t)q.mem[0].xhat & 15) == 0) {
+    const WideShape& ws = plan.w;
     const WideTile& t = kWideTiles[ws.kind];
     WideParams w{};
     for (int i = 0; i < g.count; ++i) {
@@ -734,7 +750,7 @@ static int run_group_qmm(const Group& g, const void* x, int x_type, int64_t rows
     }
     return check_launch("EXL3 QMM launch");
   }
-  const QmmShape sh = choose_qmm_shape(g.in, g.total_out, rows);
+  const QmmShape& sh = plan.q;
   q.members = g.count;
   q.partials = (float*)(scratch + xhats);
   q.counters = counters;
@@ -752,21 +768,26 @@ static int run_group_qmm(const Group& g, const void* x, int x_type, int64_t rows
   return check_launch("EXL3 QMM launch");
 }
 
+// `given`: the QMM's plan where the caller has derived it (rows > 16), or null.
 static int group_forward(const Group& g, const void* x, int x_type, int64_t rows,
-                         void* const* ys, void* ws, size_t ws_bytes, hipStream_t stream) {
+                         void* const* ys, void* ws, size_t ws_bytes, hipStream_t stream,
+                         const QmmPlan* given = nullptr) {
   if (!x) return fail(EXL3_EINVAL, "null activation pointer");
   for (int i = 0; i < g.count; ++i)
     if (!ys[i]) return fail(EXL3_EINVAL, "null activation pointer");
   if (!valid_dtype(x_type)) return fail(EXL3_EINVAL, "unsupported activation dtype code %d", x_type);
   if (int rc = check_rows(g, rows)) return rc;
-  const size_t need = kWorkspaceCounterBytes + group_scratch_min(g, rows);
+  const bool qmv = rows <= kQmvMaxRows;
+  const QmmPlan plan = qmv ? QmmPlan{} : given ? *given : plan_qmm(g, rows);
+  const size_t need = kWorkspaceCounterBytes +
+                      (qmv ? qmv_scratch(g, rows) : qmm_scratch(g, rows, plan.least));
   if (!ws || ws_bytes < need)
     return fail(EXL3_EINVAL, "workspace too small: %zu bytes given, %zu needed", ws_bytes, need);
   uint32_t* counters = (uint32_t*)ws;
   char* scratch = (char*)ws + kWorkspaceCounterBytes;
   const Glu none{};
-  if (rows <= kQmvMaxRows) return run_group_qmv(g, x, x_type, rows, ys, counters, scratch, none, stream);
-  return run_group_qmm(g, x, x_type, rows, ys, counters, scratch,
+  if (qmv) return run_group_qmv(g, x, x_type, rows, ys, counters, scratch, none, stream);
+  return run_group_qmm(g, plan, x, x_type, rows, ys, counters, scratch,
                        ws_bytes - kWorkspaceCounterBytes, nullptr, stream);
 }
 
@@ -789,22 +810,16 @@ static int mlp_check(const exl3_linear* gate, const exl3_linear* up, const exl3_
   return EXL3_OK;
 }
 
-// `least`: what a call cannot do without, else what it makes use of.
-static size_t mlp_ws_bytes(const exl3_linear* gate, const exl3_linear* up,
-                           const exl3_linear* down, int64_t rows, bool least) {
-  const exl3_linear* gu[2] = {gate, up};
-  Group g, d;
-  if (make_group(gu, 2, g) || make_group(&down, 1, d)) return 0;
-  const size_t act = align_up(sizeof(uint16_t) * (size_t)rows * gate->out);
-  size_t need;
-  if (rows <= kQmvMaxRows) {
-    need = act + std::max(group_scratch_bytes(g, rows), group_scratch_bytes(d, rows));
-  } else {
-    // down xhat + gate and up outputs
-    need = 3 * act + (least ? std::max(group_scratch_min(g, rows), align_up(group_qmm_partials_min(d, rows)))
-                            : std::max(group_scratch_bytes(g, rows), align_up(group_qmm_partials(d, rows))));
-  }
-  return kWorkspaceCounterBytes + need;
+// Workspace of the two stages at more than 16 rows, with `gu` and `dn` bytes of
+// partials: down xhat + gate and up outputs + the larger stage's scratch.
+static size_t mlp_qmm_ws(const Group& g, int64_t rows, int hidden, size_t gu, size_t dn) {
+  const size_t act = align_up(sizeof(uint16_t) * (size_t)rows * hidden);
+  return kWorkspaceCounterBytes + 3 * act + std::max(qmm_scratch(g, rows, gu), align_up(dn));
+}
+
+static size_t mlp_qmv_ws(const Group& g, const Group& d, int64_t rows, int hidden) {
+  const size_t act = align_up(sizeof(uint16_t) * (size_t)rows * hidden);
+  return kWorkspaceCounterBytes + act + std::max(qmv_scratch(g, rows), qmv_scratch(d, rows));
 }
 
 static int mlp_forward(const exl3_linear* gate, const exl3_linear* up, const exl3_linear* down,
@@ -821,7 +836,10 @@ static int mlp_forward(const exl3_linear* gate, const exl3_linear* up, const exl
   if (int rc = make_group(&down, 1, d)) return rc;
   if (int rc = check_rows(g, rows)) return rc;
   if (int rc = check_rows(d, rows)) return rc;
-  const size_t need = mlp_ws_bytes(gate, up, down, rows, true);
+  const bool qmv = rows <= kQmvMaxRows;
+  const QmmPlan gp = qmv ? QmmPlan{} : plan_qmm(g, rows), dp = qmv ? QmmPlan{} : plan_qmm(d, rows);
+  const size_t need = qmv ? mlp_qmv_ws(g, d, rows, gate->out)
+                          : mlp_qmm_ws(g, rows, gate->out, gp.least, dp.least);
   if (!ws || ws_bytes < need)
     return fail(EXL3_EINVAL, "workspace too small: %zu bytes given, %zu needed", ws_bytes, need);
   uint32_t* counters = (uint32_t*)ws;
@@ -829,7 +847,7 @@ static int mlp_forward(const exl3_linear* gate, const exl3_linear* up, const exl
   uint16_t* act = (uint16_t*)base;  // the activation (QMV) or the down xhat (QMM)
   const size_t act_bytes = align_up(sizeof(uint16_t) * (size_t)rows * gate->out);
   void* dy[1] = {y};
-  if (rows <= kQmvMaxRows) {
+  if (qmv) {
     Glu glu{};
     glu.on = 1;
     glu.out = act;
@@ -850,14 +868,14 @@ static int mlp_forward(const exl3_linear* gate, const exl3_linear* up, const exl
   void* gu_y[2] = {base + act_bytes, base + 2 * act_bytes};
   char* scratch = base + 3 * act_bytes;
   const size_t scratch_bytes = ws_bytes - kWorkspaceCounterBytes - 3 * act_bytes;
-  if (int rc = run_group_qmm(g, x, EXL3_F16, rows, gu_y, counters, scratch, scratch_bytes, nullptr,
-                             stream))
+  if (int rc = run_group_qmm(g, gp, x, EXL3_F16, rows, gu_y, counters, scratch, scratch_bytes,
+                             nullptr, stream))
     return rc;
   if (int rc = launch_gate("SwiGLU prepare launch")) return rc;
   launch_swiglu_prepare((const uint16_t*)gu_y[0], (const uint16_t*)gu_y[1], down->suh, gate->out,
                         (int)rows, act, qmm_mfma_prologue(rows, gate->out), stream);
   if (int rc = check_launch("SwiGLU prepare launch")) return rc;
-  return run_group_qmm(d, nullptr, EXL3_F16, rows, dy, counters, scratch, scratch_bytes, act,
+  return run_group_qmm(d, dp, nullptr, EXL3_F16, rows, dy, counters, scratch, scratch_bytes, act,
                        stream);
 }
 
@@ -925,7 +943,11 @@ size_t exl3_group_workspace_bytes(const exl3_linear* const* parts, int32_t count
 size_t exl3_mlp_workspace_bytes(const exl3_linear* gate, const exl3_linear* up,
                                 const exl3_linear* down, int64_t rows) {
   if (rows < 1 || mlp_check(gate, up, down)) return 0;
-  return mlp_ws_bytes(gate, up, down, rows, false);
+  const exl3_linear* gu[2] = {gate, up};
+  Group g, d;
+  if (make_group(gu, 2, g) || make_group(&down, 1, d)) return 0;
+  if (rows <= kQmvMaxRows) return mlp_qmv_ws(g, d, rows, gate->out);
+  return mlp_qmm_ws(g, rows, gate->out, plan_qmm(g, rows).partials, plan_qmm(d, rows).partials);
 }
 
 int exl3_workspace_init(void* workspace, size_t bytes, void* stream) {
@@ -941,8 +963,9 @@ int32_t exl3_linear_output_dtype(const exl3_linear* h, int32_t x_type) {
   return result_dtype(x_type, h->bias != nullptr);
 }
 
-int exl3_linear_forward(const exl3_linear* h, const void* x, int32_t x_type, int64_t rows, void* y,
-                        int32_t y_type, void* workspace, size_t workspace_bytes, void* stream) {
+static int linear_forward(const exl3_linear* h, const void* x, int32_t x_type, int64_t rows,
+                          void* y, int32_t y_type, void* workspace, size_t workspace_bytes,
+                          void* stream, const QmmPlan* given) {
   if (!h) return fail(EXL3_EINVAL, "null EXL3 linear handle");
   if (!valid_dtype(x_type)) return fail(EXL3_EINVAL, "unsupported activation dtype code %d", x_type);
   const int want = result_dtype(x_type, h->bias != nullptr);
@@ -953,7 +976,13 @@ int exl3_linear_forward(const exl3_linear* h, const void* x, int32_t x_type, int
                 y_type, want);
   Group g;
   if (int rc = make_group(&h, 1, g)) return rc;
-  return group_forward(g, x, x_type, rows, &y, workspace, workspace_bytes, (hipStream_t)stream);
+  return group_forward(g, x, x_type, rows, &y, workspace, workspace_bytes, (hipStream_t)stream,
+                       given);
+}
+
+int exl3_linear_forward(const exl3_linear* h, const void* x, int32_t x_type, int64_t rows, void* y,
+                        int32_t y_type, void* workspace, size_t workspace_bytes, void* stream) {
+  return linear_forward(h, x, x_type, rows, y, y_type, workspace, workspace_bytes, stream, nullptr);
 }
 
 size_t exl3_linear_noalloc_max_bytes(void) { return kNoAllocBytes; }
@@ -965,7 +994,10 @@ int exl3_linear_forward_noalloc(const exl3_linear* h, const void* x, int32_t x_t
   Group g;
   if (int rc = make_group(&h, 1, g)) return rc;
   if (int rc = check_rows(g, rows)) return rc;
-  const size_t need = kWorkspaceCounterBytes + group_scratch_min(g, rows);
+  const bool qmv = rows <= kQmvMaxRows;
+  const QmmPlan plan = qmv ? QmmPlan{} : plan_qmm(g, rows);
+  const size_t need = kWorkspaceCounterBytes +
+                      (qmv ? qmv_scratch(g, rows) : qmm_scratch(g, rows, plan.least));
   if (need > kNoAllocBytes)
     return fail(EXL3_EUNSUPPORTED,
                 "allocation-free EXL3 forward of %lld rows needs %zu bytes of workspace, more "
@@ -973,7 +1005,8 @@ int exl3_linear_forward_noalloc(const exl3_linear* h, const void* x, int32_t x_t
                 (long long)rows, need, kNoAllocBytes);
   void* ws = nullptr;
   if (int rc = noalloc_scratch((hipStream_t)stream, &ws)) return rc;
-  return exl3_linear_forward(h, x, x_type, rows, y, y_type, ws, kNoAllocBytes, stream);
+  return linear_forward(h, x, x_type, rows, y, y_type, ws, kNoAllocBytes, stream,
+                        qmv ? nullptr : &plan);
 }
 
 int exl3_group_forward(const exl3_linear* const* parts, int32_t count, const void* x,

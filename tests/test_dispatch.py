@@ -3,6 +3,7 @@ holds the split-K partials of the launch that it will make (no GPU needed: none 
 these calls reaches the device)."""
 
 import ctypes
+import subprocess
 
 import pytest
 
@@ -50,3 +51,78 @@ def test_pinned_qmm_shape_keeps_its_kernel(monkeypatch, linear, env, n_in, n_out
     monkeypatch.setenv("EXL3_WIDE_TILE", "1")
     monkeypatch.setenv("EXL3_WIDE_SPLITS", "2")
     assert need(rows) >= xhat_bytes(rows, n_in) + 4 * 2 * rows * n_out
+
+
+# ---------------------------------------------------------------------------
+# one derivation of the launch shape per entry point
+# ---------------------------------------------------------------------------
+COUNTER = r"""
+#include <dlfcn.h>
+#include <cstdint>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <initializer_list>
+static int reads;
+// seen by the library in place of libc's: each derivation of a QMM's launch shape
+// reads this name once
+extern "C" char* getenv(const char* name) noexcept {
+  if (!std::strcmp(name, "EXL3_QMM_MB")) ++reads;
+  static char* (*real)(const char*) = (char* (*)(const char*))dlsym(RTLD_NEXT, "getenv");
+  return real(name);
+}
+typedef void* H;
+template <class F> F sym(void* lib, const char* name) {
+  F f = (F)dlsym(lib, name);
+  if (!f) { std::printf("no %s\n", name); _Exit(2); }
+  return f;
+}
+int main(int, char** argv) {
+  void* lib = dlopen(argv[1], RTLD_NOW | RTLD_LOCAL);
+  if (!lib) { std::printf("%s\n", dlerror()); return 2; }
+  auto create = sym<int (*)(const void*, int, int, int, int, const void*, const void*, const void*, H*)>(lib, "exl3_linear_create");
+  auto lin_ws = sym<size_t (*)(H, int64_t)>(lib, "exl3_linear_workspace_bytes");
+  auto lin = sym<int (*)(H, const void*, int, int64_t, void*, int, void*, size_t, void*)>(lib, "exl3_linear_forward");
+  auto noalloc = sym<int (*)(H, const void*, int, int64_t, void*, int, void*)>(lib, "exl3_linear_forward_noalloc");
+  auto grp_ws = sym<size_t (*)(H*, int, int64_t)>(lib, "exl3_group_workspace_bytes");
+  auto grp = sym<int (*)(H*, int, const void*, int, int64_t, void**, void*, size_t, void*)>(lib, "exl3_group_forward");
+  auto mlp_ws = sym<size_t (*)(H, H, H, int64_t)>(lib, "exl3_mlp_workspace_bytes");
+  auto mlp = sym<int (*)(H, H, H, const void*, int64_t, void*, void*, size_t, void*)>(lib, "exl3_mlp_forward");
+  sym<void (*)(const char*)>(lib, "exl3_debug_fail_launch")("EXL3 QMM launch");
+  void* f = (void*)0x1000;
+  H g, u, d;
+  create(f, 4096, 14336, 4, 0, f, f, nullptr, &g);
+  create(f, 4096, 14336, 4, 0, f, f, nullptr, &u);
+  create(f, 14336, 4096, 4, 0, f, f, nullptr, &d);
+  H gu[2] = {g, u};
+  void* ys[2] = {f, f};
+  const size_t big = (size_t)1 << 40;
+  auto show = [](const char* what, int rc) { std::printf("%s %d %d\n", what, rc, reads); reads = 0; };
+  reads = 0;
+  for (int64_t rows : {20, 300, 2048}) {
+    lin_ws(g, rows), show("linear_ws", 0);
+    show("linear", lin(g, f, 9, rows, f, 9, f, big, nullptr));
+    noalloc(g, f, 9, rows, f, 9, nullptr), show("noalloc", 0);
+    grp_ws(gu, 2, rows), show("group_ws", 0);
+    show("group", grp(gu, 2, f, 9, rows, ys, f, big, nullptr));
+    mlp_ws(g, u, d, rows), show("mlp_ws", 0);
+    show("mlp", mlp(g, u, d, f, rows, f, f, big, nullptr));
+  }
+}
+"""
+
+
+def test_launch_shape_is_derived_once_per_call(tmp_path):
+    """A program whose own getenv counts how often the library looks at a tuning
+    override: every entry point derives each QMM's launch shape once (a fused MLP has
+    two QMMs).  The calls end at the armed launch gate, before any HIP call."""
+    src, exe = tmp_path / "count.cpp", tmp_path / "count"
+    src.write_text(COUNTER)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-rdynamic", "-o", str(exe), str(src), "-ldl"], check=True)
+    res = subprocess.run([str(exe), str(mlxl3_amd.LIB_PATH)], capture_output=True, text=True, timeout=120)
+    assert res.returncode == 0, res.stdout + res.stderr
+    lines = [line.split() for line in res.stdout.splitlines()]
+    assert len(lines) == 21
+    for what, rc, reads in lines:
+        assert int(rc) == (-2 if what in ("linear", "group", "mlp") else 0), (what, rc)
+        assert int(reads) == (2 if what.startswith("mlp") else 1), (what, reads)
