@@ -488,19 +488,36 @@ static size_t wide_partials(const Group& g, int64_t rows, const WideShape& w) {
 
 // Sets p.w to the fastest shape whose partials fit in `budget` bytes and p.wide to
 // whether it runs: where it is modelled faster than the producer/consumer kernel
-// (whose model leaves out ~6 us of ring fill and epilogue).  Two corrections: with
-// splits its sums take a launch more, which a call of less than ~25 us (20 in the
-// model) cannot hide from the host (us a call, producer/consumer kernel against this
-// one: 32 rows x 4096 x 3968 19.3 / 22.7, 71 x 2048 x 1536 18.6 / 21.5, 36 x 4096 x
-// 5888 21.2 / 23.0); and two MB = 1 workgroups share a CU, which the model leaves out
-// past 256 of them (18 x 22656 x 22656 142 / 152 to 170).
+// (whose model leaves out ~6 us of ring fill and epilogue).  That model's step times
+// were fitted at K = 4 with an earlier epilogue and price some launches too high; they
+// stay as they are where they choose that kernel's own shape, and are corrected here
+// (us a call with rotated weights, that kernel / this one, 11850 random shapes x rows
+// x K: of 5454 calls taken at its full price 160 lost more than 2 % against its earlier
+// form, up to 11 %; 23 of 4748 are left, and 34 of 3572 in another 8950, most of them
+// inputs of 13000 and more):
+//   * one round of MB = 4 tiles at K <= 4 against one 128 x 256 split here, which
+//     decodes every weight twice as often, 0.86: 5120 x 27648 rows 172 K = 3 87.6 / 94.4,
+//     rows 152 K = 1 83.9 / 89.3, 8960 x 28416 rows 131 K = 3 143.6 / 156.2.  At K >= 5
+//     that kernel's producers are the slower part and the model holds;
+//   * up to 64 rows in one round of MB = 1 tiles against 128 x 256, 0.9: 5120 x 27648 rows 32 K = 4
+//     51.4 / 53.9, rows 35 K = 1 50.6 / 57.0, K = 6 56.5 / 61.9;
+//   * two MB = 1 workgroups share a CU, which the model leaves out past 256 of them,
+//     0.75: 18 x 22656 x 22656 142 / 152 to 170.
+// With splits the sums take a launch more, which a call of less than ~25 us (20 in the
+// model) cannot hide from the host: 32 rows x 4096 x 3968 19.3 / 22.7, 71 x 2048 x 1536
+// 18.6 / 21.5, 36 x 4096 x 5888 21.2 / 23.0.
 static void plan_wide(const Group& g, int64_t rows, size_t budget, QmmPlan& p) {
   const int units[2] = {group_units(g, 128), group_units(g, 256)};
   p.w = choose_wide_shape(g.in, units, rows, budget);
-  const int64_t wgs = (int64_t)p.q.mtiles * (g.total_out / 128) * p.q.splits;
-  p.wide = p.forced_wide ||
-           ((p.w.splits == 1 || p.q.cost >= 20000.0) &&
-            p.w.cost < (p.q.mb == 1 && wgs > 256 ? 0.75 : 1.0) * p.q.cost + 6000.0);
+  const bool one_round = (int64_t)p.q.mtiles * (g.total_out / 128) * p.q.splits <= 256;
+  const bool tile128 = p.w.kind == 1;
+  double price = 1.0;
+  if (p.q.mb == 1)
+    price = !one_round ? 0.75 : tile128 && rows <= 64 ? 0.9 : 1.0;
+  else if (p.q.mb == 4 && one_round && tile128 && p.w.splits == 1 && g.k <= 4)
+    price = 0.86;
+  p.wide = p.forced_wide || ((p.w.splits == 1 || p.q.cost >= 20000.0) &&
+                             p.w.cost < price * p.q.cost + 6000.0);
 }
 
 // The plan of a call, derived once per entry point.  The copies of the kernel in

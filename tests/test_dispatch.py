@@ -126,3 +126,27 @@ def test_launch_shape_is_derived_once_per_call(tmp_path):
     for what, rc, reads in lines:
         assert int(rc) == (-2 if what in ("linear", "group", "mlp") else 0), (what, rc)
         assert int(reads) == (2 if what.startswith("mlp") else 1), (what, reads)
+
+
+# ---------------------------------------------------------------------------
+# the rule between the two kernels, where a split launch shows in the workspace
+# ---------------------------------------------------------------------------
+@pytest.mark.parametrize("k", [1, 2, 4, 8])
+@pytest.mark.parametrize("n_in, n_out, rows", [(5120, 27648, 17), (5120, 27648, 32), (5120, 27648, 48), (4736, 27776, 29)])
+def test_one_round_of_64_rows_keeps_the_producer_consumer_kernel(monkeypatch, linear, k, n_in, n_out, rows):
+    """Up to 64 rows in one round of workgroups: 128-row tiles in registers measured
+    2 to 11 % slower.  The producer/consumer launch has one split, no partials."""
+    need = linear(n_in, n_out, k)
+    assert need(rows) == xhat_bytes(rows, n_in)
+    monkeypatch.setenv("EXL3_WIDE", "1")
+    assert need(rows) > xhat_bytes(rows, n_in)
+
+
+@pytest.mark.parametrize("n_in, n_out, rows", [(14336, 4096, 300), (14336, 4096, 200), (8192, 8192, 200)])
+def test_long_inputs_stay_in_registers(monkeypatch, linear, n_in, n_out, rows):
+    need = linear(n_in, n_out)
+    got = need(rows)
+    monkeypatch.setenv("EXL3_WIDE", "1")
+    assert got == need(rows)
+    monkeypatch.setenv("EXL3_WIDE", "0")
+    assert got != need(rows)
