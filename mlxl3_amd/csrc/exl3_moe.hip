@@ -93,36 +93,53 @@ int moe_splits(const exl3_moe* h, int64_t slots, int block_rows, int k_in, int c
   return std::max(1, std::min(s, k_in / 128));
 }
 
-// Whether the grouped expert QMMs run as moe_wide_kernel: where its blocks (160
-// rows, 128 at K = 8) decode an expert's weights at most half as often as
-// moe_mm_kernel's 64-row blocks on the average rows per expert.  Measured (us, old ->
-// new; rows per expert): 128 experts top-8 K = 3, 2048x768: 62 264 -> 298, 125 451 ->
-// 376, 250 825 -> 739; 64 experts top-6 K = 4, 2048x1024: 56 168 -> 188, 188 406 -> 425;
-// 8 experts top-2: 64 80 -> 87, 250 132 -> 106, 1000 268 -> 242; 32 experts top-4 K = 5,
-// 3072x1536: 125 362 -> 264.  Not where the last round of two workgroups per CU would be
-// mostly empty (8 experts, 687 rows each: 1.25 rounds, 195 -> 202), and for GELU, whose
-// glue in a launch of its own costs more (its binary64 tanh), only above 112 rows per
-// expert (70 364 -> 384, 113 487 -> 479, 125 524 -> 500).  Its copies address the bank and the gathered rows with
-// 32-bit byte offsets, 16 bytes at a time.  Pinned split counts (one split among them:
-// a row of such a bank has the same bits in every call) or block rows keep
-// moe_mm_kernel.  EXL3_MOE_WIDE=0/1 forces it off or on (tuning).
-bool moe_takes_wide(const exl3_moe* h, int64_t slots) {
+// Which kernel the grouped expert QMMs run as: moe_mm_kernel, moe_wide_kernel, or
+// either one by the blocks that the call's routes cut, which only the device knows
+// (both are launched; the plan gives one of them every block, the other none).
+// Blocks of 160 rows (128 at K = 8) pay where they decode an expert's weights about
+// half as often as blocks of 64.  On the average rows per expert the host asks for
+// that, for more than 64 of them, and for no mostly empty last round of two workgroups
+// per CU.  But routes are not even: with a bias of N(0, 0.5) per expert on the logits,
+// 112 to 128 rows per expert at K <= 4 ran at 1.09 of moe_mm_kernel's time (0.89 even),
+// at worst 1.36.  The blocks of both sizes tell: of 6696 calls (1024..4096 x 512..2048, 8
+// to 128 experts, 40 to 1200 rows each, even and uneven), time against moe_mm_kernel by
+// the ratio of their counts, SiLU:
+//   K <= 2   1.6-1.8 1.10-1.18   1.9-2.0 1.02   2.0-2.1 0.98   2.1-2.2 0.94   more 0.89
+//   K = 3, 4 1.6-1.8 1.09   1.9-2.0 0.93 even, 1.04 uneven   2.0-2.1 0.92   more 0.89
+//   K = 5, 6 1.5-1.7 0.98   1.7-1.8 0.95   1.9-2.0 0.85   more 0.80
+//   K = 8    0.87 at worst, so always
+// GELU, whose glue in a launch of its own costs more (its binary64 tanh), above 112
+// rows per expert: K <= 4 never (1.09 at 2.0-2.1, 1.00 above 2.2), K = 5, 6 from 2.0 on
+// (0.92 even, 0.98 uneven), K = 8 always.
+// The copies of moe_wide_kernel address the bank and the gathered rows with 32-bit byte
+// offsets, 16 bytes at a time.  Pinned split counts (one split among them: a row of such
+// a bank has the same bits in every call) or block rows keep moe_mm_kernel.
+// EXL3_MOE_WIDE=0/1 forces it off or on (tuning).
+enum MoeWideMode { kMoeNarrow, kMoeWideOnly, kMoeByBlocks };
+MoeWideMode moe_wide_mode(const exl3_moe* h, int64_t slots) {
   const int64_t bank = std::max((int64_t)2 * h->experts * h->hidden / 8 * h->k * h->in,
                                 (int64_t)h->experts * h->in / 8 * h->k * h->hidden);
   const int64_t rows = std::max(2 * slots * h->in, slots * h->hidden) * 2;
-  if (bank >= ((int64_t)1 << 32) || rows >= ((int64_t)1 << 32)) return false;
-  if (((uintptr_t)h->gu_trellis | (uintptr_t)h->down_trellis) & 15) return false;
+  if (bank >= ((int64_t)1 << 32) || rows >= ((int64_t)1 << 32)) return kMoeNarrow;
+  if (((uintptr_t)h->gu_trellis | (uintptr_t)h->down_trellis) & 15) return kMoeNarrow;
   // the gate's and up's sums borrow the slot outputs' buffer (f32 rows of `in`)
-  if (h->hidden > h->in || h->hidden / 128 > 65535) return false;
-  if (h->force_splits > 0 || getenv("EXL3_MOE_BLOCK_ROWS")) return false;
-  if (const char* env = getenv("EXL3_MOE_WIDE")) return atoi(env) != 0;
+  if (h->hidden > h->in || h->hidden / 128 > 65535) return kMoeNarrow;
+  if (h->force_splits > 0 || getenv("EXL3_MOE_BLOCK_ROWS")) return kMoeNarrow;
+  if (const char* env = getenv("EXL3_MOE_WIDE")) return atoi(env) != 0 ? kMoeWideOnly : kMoeNarrow;
+  if (h->gelu && h->k <= 4) return kMoeNarrow;
   const int64_t avg = slots / h->experts, rows_wide = moe_wide_rows(h->k);
-  if (avg <= (h->gelu ? 112 : 64)) return false;
+  if (avg <= (h->gelu ? 112 : 64)) return kMoeNarrow;
   const int64_t blocks = (avg + rows_wide - 1) / rows_wide;
-  if ((avg + 63) / 64 < 2 * blocks) return false;
+  if ((avg + 63) / 64 < 2 * blocks) return kMoeNarrow;
   const int64_t wgs = h->experts * blocks * (2 * h->hidden / 128), slots_cu = 512;  // two per CU
   const int64_t rounds = (wgs + slots_cu - 1) / slots_cu;
-  return rounds == 1 || 4 * wgs >= 3 * rounds * slots_cu;
+  if (rounds > 1 && 4 * wgs < 3 * rounds * slots_cu) return kMoeNarrow;
+  return h->k == 8 ? kMoeWideOnly : kMoeByBlocks;
+}
+
+// kMoeByBlocks: blocks of 64 rows per block of 160 from which the latter run, in tenths.
+int moe_wide_tenths(const exl3_moe* h) {
+  return h->gelu || h->k <= 2 ? 20 : h->k <= 4 ? 19 : 17;
 }
 
 // The small-row path (decode): up to this many routed slots run as two
@@ -159,7 +176,8 @@ int moe_small_splits(const exl3_moe* h, int64_t slots, int k_in, int col_blocks,
 struct MoeLayout {
   size_t counts, rank, sorted, expert_count, table, counters, xgu, xd, z, partials, total;
   int max_blocks, ncounters, splits_gu, splits_down, block_rows;
-  int wide;                         // the expert QMMs of exl3_moe_wide.hpp
+  MoeWideMode wide;                 // the expert QMMs of exl3_moe_wide.hpp
+  int wide_blocks;                  // bound of their blocks
   int small, small_gu, small_down;  // small-row path and its split counts
 };
 
@@ -178,8 +196,8 @@ bool moe_layout(const exl3_moe* h, int64_t rows, MoeLayout& L) {
     const int v = atoi(env);
     if (v == 16 || v == 32 || v == 64) L.block_rows = v;
   }
-  L.wide = moe_takes_wide(h, slots);
-  if (L.wide) L.block_rows = moe_wide_rows(h->k);
+  L.wide = moe_wide_mode(h, slots);
+  if (L.wide == kMoeWideOnly) L.block_rows = moe_wide_rows(h->k);
   // each routed expert's last block may be partial: sum ceil(c_e/b) <=
   // slots/b + (experts routed) <= slots/b + min(E, slots).  The expert QMM
   // grids are sized by this bound, so a decode call (8 slots) launches the
@@ -189,8 +207,14 @@ bool moe_layout(const exl3_moe* h, int64_t rows, MoeLayout& L) {
   if (ncounters > INT32_MAX) return false;
   L.max_blocks = (int)max_blocks;
   L.ncounters = (int)ncounters;
-  L.splits_gu = L.wide ? 1 : moe_splits(h, slots, L.block_rows, h->in, h->hidden / 128);
-  L.splits_down = L.wide ? 1 : moe_splits(h, slots, L.block_rows, h->hidden, h->in / 128);
+  // chosen by the blocks, they are 10 / tenths of the others at the most
+  L.wide_blocks = L.max_blocks;
+  if (L.wide == kMoeByBlocks)
+    L.wide_blocks = std::min((int)(slots / moe_wide_rows(h->k) + std::min<int64_t>(h->experts, slots) + 1),
+                             10 * L.max_blocks / moe_wide_tenths(h));
+  const bool narrow = L.wide != kMoeWideOnly;
+  L.splits_gu = narrow ? moe_splits(h, slots, L.block_rows, h->in, h->hidden / 128) : 1;
+  L.splits_down = narrow ? moe_splits(h, slots, L.block_rows, h->hidden, h->in / 128) : 1;
   // small-row path: its arrival counters (gate/up, down, top-k sums) must fit
   // the workspace's counter region
   const int64_t small_counters =
@@ -211,7 +235,7 @@ bool moe_layout(const exl3_moe* h, int64_t rows, MoeLayout& L) {
     off = moe_align(off + bytes);
     return at;
   };
-  L.counts = take(2 * sizeof(int));
+  L.counts = take(3 * sizeof(int));
   L.rank = take((size_t)slots * sizeof(int));
   L.sorted = take((size_t)slots * sizeof(int));
   L.expert_count = take((size_t)h->experts * sizeof(int));
@@ -422,6 +446,8 @@ int exl3_moe_forward(const exl3_moe* h, const void* x, int32_t x_type, int64_t r
   pp.counters = (uint32_t*)(ws + L.counters);
   pp.ncounters = L.ncounters;
   pp.block_rows = L.block_rows;
+  pp.alt_rows = L.wide == kMoeByBlocks ? moe_wide_rows(h->k) : 0;
+  pp.alt_tenths = moe_wide_tenths(h);
   MoeGatherParams gp;
   gp.x = x;
   gp.x_dtype = x_type;
@@ -436,7 +462,7 @@ int exl3_moe_forward(const exl3_moe* h, const void* x, int32_t x_type, int64_t r
       1u + (unsigned)((2 * (int64_t)slots * ((h->in / 128 + 7) / 8) + 3) / 4);
   const size_t plan_lds = (3 * (size_t)h->experts + 1) * sizeof(int);
   if (int rc = launch_gate("moe plan")) return rc;
-  if (L.wide)
+  if (L.wide != kMoeNarrow)
     launch_moe_route16(pp, gp, plan_lds, s);
   else if ((((uintptr_t)x | (uintptr_t)h->gu_suh) & 15) == 0)
     moe_route_kernel<true><<<route_wgs, 256, plan_lds, s>>>(pp, gp);
@@ -481,11 +507,15 @@ int exl3_moe_forward(const exl3_moe* h, const void* x, int32_t x_type, int64_t r
   d.scores = scores;
   d.scores_dtype = scores_type;
   d.z = ws + L.z;
-  if (L.wide) {
+  if (L.wide != kMoeNarrow) {
     const MoeWideFn wide = kMoeWide[h->k - 1][h->cb];
-    if (int rc = wide(q, true, grid_blocks, (uint16_t*)d.z, s)) return rc;
-    if (int rc = wide(d, false, grid_blocks, nullptr, s)) return rc;
-  } else {
+    const int wide_blocks = (L.wide_blocks + 7) / 8 * 8;
+    MoeMmParams wq = q, wd = d;
+    if (L.wide == kMoeByBlocks) wq.counts = wd.counts = pp.counts + 2;
+    if (int rc = wide(wq, true, wide_blocks, (uint16_t*)d.z, s)) return rc;
+    if (int rc = wide(wd, false, wide_blocks, nullptr, s)) return rc;
+  }
+  if (L.wide != kMoeWideOnly) {
     gateup<<<grid_blocks * q.col_blocks * q.splits, 512, 0, s>>>(q);
     if (int rc = check_launch("moe gate/up")) return rc;
     down<<<grid_blocks * d.col_blocks * d.splits, 256, 0, s>>>(d);

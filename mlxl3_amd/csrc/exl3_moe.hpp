@@ -47,21 +47,26 @@ struct MoePlanParams {
   int* rank;                 // [slots] scratch
   int* sorted_slot;          // [slots] slot at each sorted position
   int4* table;               // [max_blocks] (expert, first sorted position, rows, 0)
-  int* counts;               // [2]: block-table entries, routed slots
+  int* counts;               // [3]: entries of block_rows rows, routed slots, entries of
+                             // alt_rows rows (one of the two entry counts is 0)
   int* expert_count;         // [experts] (rows routed to each expert)
   uint32_t* counters;        // [ncounters] tile arrival counters, cleared here
   int ncounters;
-  int block_rows;            // 16, 32 or 64
+  int block_rows;            // 16, 32 or 64; 128 or 160 for moe_wide_kernel alone
+  int alt_rows, alt_tenths;  // 0, or: blocks of alt_rows (128 or 160) rows where those of
+                             // block_rows are at least alt_tenths / 10 times as many
 };
 
 // The route plan, run by one workgroup of NT threads: counting sort of the
 // slots by expert, exclusive scans of the per-expert row and block counts,
 // the block table.  Slots with an expert id >= experts are left out (their
-// contribution is zero).  LDS (dynamic): cnt[E], off[E], boff[E+1].
+// contribution is zero).  With alt_rows the blocks' size follows from the counts
+// of both (the rule and its figures: moe_wide_mode).  LDS (dynamic): cnt[E], off[E],
+// boff[E+1].
 template <int NT>
 __device__ __forceinline__ void moe_plan_block(const MoePlanParams& p) {
   extern __shared__ int lds[];
-  __shared__ int wsum[2][NT / 64];
+  __shared__ int wsum[3][NT / 64];
   int* cnt = lds;
   int* off = lds + p.experts;
   int* boff = lds + 2 * p.experts;
@@ -88,33 +93,41 @@ __device__ __forceinline__ void moe_plan_block(const MoePlanParams& p) {
   // each thread writes its run's offsets
   const int per = (p.experts + NT - 1) / NT;
   const int e0 = min(tid * per, p.experts), e1 = min(e0 + per, p.experts);
-  int lc = 0, lb = 0;
+  const int alt_rows = p.alt_rows ? p.alt_rows : p.block_rows;
+  int lc = 0, lb = 0, la = 0;
   for (int e = e0; e < e1; ++e) {
     lc += cnt[e];
     lb += (cnt[e] + p.block_rows - 1) / p.block_rows;
+    la += (cnt[e] + alt_rows - 1) / alt_rows;
   }
-  int ic = lc, ib = lb;  // inclusive scan inside the wave
+  int ic = lc, ib = lb, ia = la;  // inclusive scan inside the wave
   const int lane = tid & 63, wv = tid >> 6;
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
-    const int tc = __shfl_up(ic, d, 64), tb = __shfl_up(ib, d, 64);
-    if (lane >= d) ic += tc, ib += tb;
+    const int tc = __shfl_up(ic, d, 64), tb = __shfl_up(ib, d, 64), ta = __shfl_up(ia, d, 64);
+    if (lane >= d) ic += tc, ib += tb, ia += ta;
   }
-  if (lane == 63) wsum[0][wv] = ic, wsum[1][wv] = ib;
+  if (lane == 63) wsum[0][wv] = ic, wsum[1][wv] = ib, wsum[2][wv] = ia;
   __syncthreads();
+  int all_b = 0, all_a = 0;  // the whole call's blocks of either size
+  for (int w = 0; w < NT / 64; ++w) all_b += wsum[1][w], all_a += wsum[2][w];
+  const bool alt = p.alt_rows && 10 * all_b >= p.alt_tenths * all_a;  // uniform
+  const int block_rows = alt ? alt_rows : p.block_rows;
+  if (alt) ib = ia, lb = la;
   int bc = 0, bb = 0;
-  for (int w = 0; w < wv; ++w) bc += wsum[0][w], bb += wsum[1][w];
+  for (int w = 0; w < wv; ++w) bc += wsum[0][w], bb += wsum[alt ? 2 : 1][w];
   int rc = bc + ic - lc, rb = bb + ib - lb;  // exclusive prefix of this run
   for (int e = e0; e < e1; ++e) {
     off[e] = rc;
     boff[e] = rb;
     rc += cnt[e];
-    rb += (cnt[e] + p.block_rows - 1) / p.block_rows;
+    rb += (cnt[e] + block_rows - 1) / block_rows;
   }
   if (tid == NT - 1) {
     boff[p.experts] = rb;
-    p.counts[0] = rb;
+    p.counts[0] = alt ? 0 : rb;
     p.counts[1] = rc;
+    p.counts[2] = alt ? rb : 0;
   }
   __syncthreads();
   for (int s0 = tid; s0 < p.slots; s0 += kPlanBatch * NT) {
@@ -135,8 +148,8 @@ __device__ __forceinline__ void moe_plan_block(const MoePlanParams& p) {
   for (int e = tid; e < p.experts; e += NT) {
     p.expert_count[e] = cnt[e];
     for (int b = boff[e]; b < boff[e + 1]; ++b) {
-      const int first = off[e] + (b - boff[e]) * p.block_rows;
-      p.table[b] = make_int4(e, first, min(p.block_rows, off[e] + cnt[e] - first), 0);
+      const int first = off[e] + (b - boff[e]) * block_rows;
+      p.table[b] = make_int4(e, first, min(block_rows, off[e] + cnt[e] - first), 0);
     }
   }
 }

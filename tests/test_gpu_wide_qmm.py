@@ -227,3 +227,119 @@ def test_moe_wide_unaligned_input(monkeypatch, dtype):
     assert buf.data_ptr() % 16 != 0
     a, b = moe.forward(t, sel, sc), moe.forward(buf, sel, sc)
     assert torch.equal(a.float(), b.float())
+
+
+def routes_of(counts, top_k, seed, idle=0):
+    """selected [rows, top_k] that gives expert e counts[e] slots, in random order;
+    the ids from len(counts) on are `idle` slots outside the bank."""
+    ids = np.concatenate([np.repeat(np.arange(len(counts)), counts), np.full(idle, len(counts))])
+    assert ids.size % top_k == 0
+    np.random.default_rng(seed).shuffle(ids)
+    return ids.reshape(-1, top_k).astype(np.uint32)
+
+
+# 16 experts, mean rows per expert above the 64 (GELU: 112) from which the host lets
+# the device choose; wide: blocks of 160 rows are at least 2 (K = 3, 4 with SiLU: 1.9, K
+# = 5, 6: 1.7) times fewer than blocks of 64
+CHOICES = [
+    # counts, k, activation, idle slots, wide
+    ([80] * 16, 1, "silu", 0, True),                  # 32 against 16 blocks
+    ([80] * 16, 4, "silu", 0, True),
+    ([80] * 15 + [64], 4, "silu", 0, True),           # 31 against 16: 1.94
+    ([80] * 14 + [64, 64], 4, "silu", 0, False),      # 30 against 16: 1.88
+    ([80] * 15 + [64], 2, "silu", 0, False),          # 1.94 < 2
+    ([160] * 8 + [64] * 8, 3, "silu", 0, True),       # 32 against 16
+    ([161] * 8 + [64] * 8, 3, "silu", 8, False),      # 32 against 24
+    ([30, 130] * 8, 4, "silu", 0, True),              # 1 + 3 against 1 + 1
+    ([30, 120] * 8, 4, "silu", 0, False),             # 1 + 2 against 1 + 1
+    ([30, 120] * 8, 5, "silu", 0, False),             # 1.5 < 1.7
+    ([1, 0, 1279] + [0] * 13, 3, "silu", 0, True),    # 21 against 9, idle experts
+    ([1, 0, 1279] + [0] * 13, 6, "silu", 16, True),   # ids outside the bank
+    ([60] * 12 + [200] * 4, 6, "silu", 0, False),     # 28 against 20: 1.4
+    ([120] * 16, 4, "gelu", 0, False),                # GELU banks of K <= 4 never
+    ([120] * 16, 5, "gelu", 0, True),
+    ([128] * 15 + [64], 6, "gelu", 0, False),       # 31 against 16 < 2
+    ([30, 130] * 8, 8, "silu", 0, None),              # K = 8: always, nothing to choose
+]
+
+
+@pytest.mark.parametrize("case_id", range(len(CHOICES)))
+def test_moe_block_choice_follows_the_routes(monkeypatch, case_id):
+    """Whether the experts run in blocks of 160 rows is decided from the blocks that the
+    call's routes really cut, on the device: one of the two kernels gets every block,
+    the other none.  The output matches the oracle and both forced forms either way."""
+    import test_gpu_moe as m
+    import torch
+
+    counts, k, act, idle, wide = CHOICES[case_id]
+    print(f"moe choice {case_id} k={k} {act}", flush=True)
+    layer, _, _, _ = m.case(256, 128, 16, 2, 4, k, 760)
+    sel = routes_of(counts, 2, 761 + case_id, idle)
+    rows = sel.shape[0]
+    x = synth.activations(762, case_id, rows, 256)
+    _, sc = synth.moe_routes(763, 1, rows, 16, 2)
+    moe = m.make_moe(layer, 2, k, 0, activation=act)
+    y = m.run(moe, x, sel, sc)
+    narrow_blocks, routed, wide_blocks = moe._ws.buf[65536:65536 + 12].view(torch.int32).tolist()
+    b64 = sum(-(-c // 64) for c in counts)
+    bw = sum(-(-c // 160) for c in counts)
+    assert routed == sum(counts)
+    if wide is not None:
+        assert (narrow_blocks, wide_blocks) == ((0, bw) if wide else (b64, 0))
+    pick = np.arange(case_id % 5, rows, 11)
+    inside = (sel[pick] < 16).all(1)
+    pick = pick[inside]
+    ref = oracle.moe_forward(x[pick], sel[pick], sc[pick], *layer, k, 0, activation=act)
+    m.check(y[pick], ref, f"choice {case_id}")
+    # two outputs that may each be TOL away from the oracle are at most twice that apart
+    rms = np.sqrt(np.mean(y.astype(np.float64) ** 2))
+    for forced in "01":
+        monkeypatch.setenv("EXL3_MOE_WIDE", forced)
+        gap = m.run(moe, x, sel, sc).astype(np.float64) - y
+        assert np.sqrt(np.mean(gap ** 2)) <= 2 * m.TOL_REL * rms, (case_id, forced)
+        assert np.abs(gap).max() <= 2 * m.TOL_RMS * rms, (case_id, forced)
+
+
+def test_moe_choice_alternates_on_one_workspace():
+    """Even and uneven routes in turn on one operator (one workspace): each call equals
+    its first result bit for bit, so neither kernel reads what the other left."""
+    import test_gpu_moe as m
+    import torch
+
+    layer, _, _, _ = m.case(512, 256, 16, 2, 4, 4, 770)
+    moe = m.make_moe(layer, 2, 4, 0)
+    ins = []
+    for i, counts in enumerate(([80] * 16, [30, 130, 30, 90] * 4, [30, 120] * 8)):
+        sel = routes_of(counts, 2, 771 + i)
+        x = synth.activations(772, i, sel.shape[0], 512)
+        _, sc = synth.moe_routes(773, i, sel.shape[0], 16, 2)
+        ins.append((m.dev(x), m.dev(sel), m.dev(sc)))
+    want = [moe.forward(*a).clone() for a in ins]
+    outs = [moe.forward(*ins[i % 3]) for i in range(30)]
+    torch.cuda.synchronize()
+    for i, y in enumerate(outs):
+        assert torch.equal(y.view(torch.int16), want[i % 3].view(torch.int16)), i
+
+
+@pytest.mark.parametrize("experts", [3840, 4096])
+def test_moe_wide_largest_bank(monkeypatch, experts):
+    """The most experts a bank may have: the route launch's histogram next to its gather
+    rows is the largest LDS request there is (66 KB)."""
+    import test_gpu_moe as m
+    import torch
+
+    print(f"moe wide {experts} experts", flush=True)
+    g = torch.Generator().manual_seed(experts)
+    t = lambda *s: torch.randint(-32768, 32768, s, dtype=torch.int16, generator=g).cuda()
+    f = lambda *s: ((torch.rand(*s, generator=g) + 0.5) / 12).half().cuda()
+    import mlxl3_amd
+
+    moe = mlxl3_amd.Exl3SwitchGlu(t(8, 2 * experts * 8, 16), f(experts, 2, 128), f(experts, 2, 128),
+                                  t(8, experts * 8, 16), f(experts, 128), f(experts, 128), top_k=2, k=1, cb=0)
+    x = torch.randn(60, 128, generator=g).half().cuda()
+    sel = torch.randint(0, experts, (60, 2), generator=g).int().cuda()
+    sc = torch.rand(60, 2, generator=g).half().cuda()
+    monkeypatch.setenv("EXL3_MOE_WIDE", "1")
+    y = moe.forward(x, sel, sc).cpu().numpy()
+    monkeypatch.setenv("EXL3_MOE_WIDE", "0")
+    m.check(y, moe.forward(x, sel, sc).cpu().numpy(), "vs the 64-row blocks")
