@@ -339,7 +339,7 @@ static size_t qmm_partial_bytes(const QmmShape& sh, int out) {
 // rows 64/768/2048 32.3/146/285 -> 29.7/105/230; that kernel keeps most launches of
 // few tiles (2048x1536 rows 256..2048 19.3-37.1 against 20.4-37.4, 4096x4096 rows 256
 // 29.3 against 30.7), where 256-column tiles leave CUs idle.
-struct WideShape {
+struct WideLaunch {
   int kind, mtiles, splits;  // kind: index of kWide and kWideTiles
   double cost;
 };
@@ -358,12 +358,12 @@ static size_t wide_partial_bytes(const WideTile& t, int64_t rows, int units, int
 
 // The cheapest shape whose partials fit in `budget` bytes (one split always fits);
 // units[i]: column units of the launch in tiles of 128 (0) or 256 (1) columns.
-static WideShape choose_wide_shape(int in, const int (&units)[2], int64_t rows, size_t budget) {
+static WideLaunch choose_wide_shape(int in, const int (&units)[2], int64_t rows, size_t budget) {
   const int nq = in / 64;
   int force_kind = -1, force_splits = 0;
   if (const char* env = getenv("EXL3_WIDE_TILE")) force_kind = std::max(0, std::min(atoi(env), 2));
   if (const char* env = getenv("EXL3_WIDE_SPLITS")) force_splits = std::max(0, atoi(env));
-  WideShape best{2, (int)((rows + 255) / 256), 1, 1e300};
+  WideLaunch best{2, (int)((rows + 255) / 256), 1, 1e300};
   for (int kind = 0; kind < 3; ++kind) {
     if (force_kind >= 0 && kind != force_kind) continue;
     const WideTile& t = kWideTiles[kind];
@@ -379,7 +379,7 @@ static WideShape choose_wide_shape(int in, const int (&units)[2], int64_t rows, 
       const double step = wgs <= 256 ? t.alone_ns : t.step_ns;
       double cost = t.fixed_ns + (double)rounds * ((nq + sp - 1) / sp) * step;
       if (sp > 1) cost += 3000.0 + 0.42 / 1024 * (double)part;
-      if (cost < best.cost) best = WideShape{kind, (int)mt, sp, cost};
+      if (cost < best.cost) best = WideLaunch{kind, (int)mt, sp, cost};
       if (force_splits) break;
     }
   }
@@ -475,13 +475,13 @@ static int group_units(const Group& g, int cols) {
 // What a QMM over the group runs (rows > 16).
 struct QmmPlan {
   QmmShape q;       // the producer/consumer kernel's shape
-  WideShape w;      // the shape in registers (exl3_wide.hpp), if that may run
+  WideLaunch w;      // the shape in registers (exl3_wide.hpp), if that may run
   bool may_wide, forced_wide, wide;  // wide: it does
   size_t least;     // bytes of partials that every workspace has to hold
   size_t partials;  // ... and that the launch takes when it is given
 };
 
-static size_t wide_partials(const Group& g, int64_t rows, const WideShape& w) {
+static size_t wide_partials(const Group& g, int64_t rows, const WideLaunch& w) {
   const WideTile& t = kWideTiles[w.kind];
   return wide_partial_bytes(t, rows, group_units(g, 32 * t.nw), w.splits);
 }
@@ -743,7 +743,7 @@ static int run_group_qmm(const Group& g, QmmPlan plan, const void* x, int x_type
   const size_t xhats = given_xhat ? 0 : g.count * xbytes;
   fit_plan(g, rows, scratch_bytes - xhats, plan);
   if (plan.wide && ((uintptr_t)q.mem[0].xhat & 15) == 0) {
-    const WideShape& ws = plan.w;
+    const WideLaunch& ws = plan.w;
     const WideTile& t = kWideTiles[ws.kind];
     WideParams w{};
     for (int i = 0; i < g.count; ++i) {

@@ -48,7 +48,7 @@ void launch_moe_route16(const MoePlanParams& pp, const MoeGatherParams& gp, size
 
 // xhat of `members` (suh, xhat) pairs of p in one launch.
 void launch_prologue(const PrologueParams& p, int members, hipStream_t s);
-// The same for the QMM (more than 16 rows): the Hadamard by MFMA.
+// The same with the Hadamard by MFMA, for large QMMs.
 void launch_prologue16(const PrologueParams& p, int members, hipStream_t s);
 // Sums the split-K partials of a kWide launch with 32*NW columns per workgroup and
 // finishes its outputs.

@@ -71,7 +71,6 @@ struct WideParams {
   WideMember mem[kMaxMembers];
   int members;
   float* partials;     // [splits][units][row blocks][16 x 32*NW f32 in fragment order]
-  uint32_t* counters;  // [mtiles * pairs], zero between calls (splits > 1)
   int in, M, x_dtype;
   int units;   // column units of all members
   int mtiles;  // ceil(M / rows per workgroup)

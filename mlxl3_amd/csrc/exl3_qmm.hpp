@@ -194,8 +194,9 @@ __device__ __forceinline__ void store8(half8 v, uint16_t* dst) {
 
 // The QMM's prologue: prologue_kernel's values with the Hadamard by MFMA, one wave
 // per 16 rows x 128 columns (~30 -> ~9 VALU instructions per element).  Only for
-// more than 16 rows: the MFMA's f32 sums may round otherwise than the butterflies'
-// in rare cases, and a row of the QMV has one value whichever launch computes it.
+// QMMs (from 2048 waves on: qmm_mfma_prologue): the MFMA's f32 sums may round otherwise
+// than the butterflies', and a row of the QMV has one value whichever launch computes
+// it.
 // grid (ceil(ceil(rows / 16) * blocks / 4), members), 256 threads.
 template <bool VEC>
 __global__ __launch_bounds__(256) void prologue16_kernel(PrologueParams p) {
@@ -356,6 +357,8 @@ __device__ __forceinline__ void qmm_finish16(uint16_t* ys, int stride, const uin
                                              const QmmOut& out, int x_dtype, size_t yoff,
                                              size_t ystride, int r0 = 0) {
   const int g = lane >> 4, n = lane & 15;
+  // h16_row<true>, written out: called, it gives qmm_kernel other registers, and 4096 x
+  // 14336 at 512 rows takes 77.7 us instead of 75.6
   half4 hm;  // H16 row n at the true columns of positions 4g + i
 #pragma unroll
   for (int i = 0; i < 4; ++i) {

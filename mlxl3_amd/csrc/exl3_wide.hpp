@@ -83,12 +83,15 @@ __device__ __forceinline__ WideSource wide_source(const void* base, size_t bytes
 // Lane l copies the 16 bytes at src + soff + off to LDS bytes lds + add + 16l
 // (soff, lds, add uniform).  The compiler sees neither the load nor the LDS
 // write: the caller waits (vmcnt) before the barrier that publishes the bytes.
+// m0 is a reserved register, which a clobber list may not name; the compiler writes it
+// only right before an instruction of its own that reads it, and the kernels that
+// copy this way have none.
 __device__ __forceinline__ void wide_copy(const u32x4& rsrc, uint32_t off, uint32_t soff,
                                           uint32_t lds, uint32_t add) {
   asm volatile("s_add_u32 m0, %3, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
                :
                : "v"(off), "s"(rsrc), "s"(soff), "s"(lds), "s"(add)
-               : "memory", "scc", "m0");
+               : "memory", "scc");
 }
 
 // The windows of states S, S + 1 of a lane into src (shared windows are taken
@@ -463,7 +466,6 @@ __global__ __launch_bounds__(64 * NW) void wide_qmm_kernel(WideParams p) {
   const bool whole = NW == 4 || pl * 256 + 128 < mm.out;
   const int nq_all = p.in >> 6;
   const int qa = split * nq_all / p.splits, nq = (split + 1) * nq_all / p.splits - qa;
-  const int tile = mtile * p.units + unit;
   const int row0 = mtile * C::kRows;
 
   if (threadIdx.x < C::kCols) {
