@@ -403,7 +403,8 @@ def test_split_exchange_alternating_inputs(n_in, n_out, rows):
     store landed would be the previous call's, so calls alternate between two
     inputs on one workspace (the previous call's partials always differ): 60
     calls, each bit-identical to its input's first result.  Shapes: the
-    single-row, row-major, fragment-order and QMM (4 K-splits) exchanges."""
+    single-row, row-major and fragment-order exchanges, and a split launch of the QMM
+    in registers, whose sums are a launch of their own."""
     torch = torch_mod()
     lin, _ = make_layer(4100 + rows, n_in, n_out, 4, 0)
     xs = [torch.from_numpy(synth.activations(60 + i, rows, rows, n_in)).cuda() for i in range(2)]
@@ -416,3 +417,26 @@ def test_split_exchange_alternating_inputs(n_in, n_out, rows):
     for i, y in enumerate(outs):
         assert torch.equal(y.view(torch.int16), want[i % 2].view(torch.int16)), i
 
+
+@pytest.mark.parametrize("n_in,n_out,rows,splits", [
+    (14336, 4096, 512, 4), (14336, 4096, 47, 8), (4096, 4096, 200, 4), (5120, 640, 100, 8),
+])
+def test_qmm_exchange_alternating_inputs(n_in, n_out, rows, splits, monkeypatch):
+    """test_split_exchange_alternating_inputs for the producer/consumer QMM, whose last
+    arriving workgroup sums the split-K partials: that kernel forced on, with the split
+    counts that its launches of few tiles take."""
+    torch = torch_mod()
+    monkeypatch.setenv("EXL3_WIDE", "0")
+    monkeypatch.setenv("EXL3_QMM_SPLITS", str(splits))
+    lin, _ = make_layer(4200 + rows, n_in, n_out, 4, 0)
+    xs = [torch.from_numpy(synth.activations(60 + i, rows, rows, n_in)).cuda() for i in range(2)]
+    ws = torch.zeros(lin.workspace_bytes(rows), dtype=torch.uint8, device="cuda")
+    # the partials of every split are in the workspace: the exchange is there
+    assert ws.numel() >= 65536 + 2 * rows * n_in + 4 * splits * rows * n_out
+    want = [lin.forward(x, workspace=ws).clone() for x in xs]
+    torch.cuda.synchronize()
+    assert not torch.equal(want[0], want[1])
+    outs = [lin.forward(xs[i % 2], workspace=ws) for i in range(60)]
+    torch.cuda.synchronize()
+    for i, y in enumerate(outs):
+        assert torch.equal(y.view(torch.int16), want[i % 2].view(torch.int16)), i

@@ -28,15 +28,14 @@ def force(monkeypatch, r, splits):
 @pytest.mark.parametrize("r", [4, 8, 16])
 def test_every_k_and_codebook(monkeypatch, k, cb, r):
     # 384 columns: the second pair holds one 128-column block; 33 rows past a tile
-    # of 16*r; 5 steps a split, one more in the last
-    n_in, n_out, rows = 704, 384, 16 * r + 33
-    n_in = n_in // 128 * 128
+    # of 16*r; 20 steps in splits of 6, 7 and 7
+    n_in, n_out, rows = 1280, 384, 16 * r + 33
     print(f"wide k={k} cb={cb} r={r}", flush=True)
     lin, (tr, suh, svh, _) = make_layer(4000 + 10 * k + cb, n_in, n_out, k, cb)
     x = synth.activations(5, k, rows, n_in)
     ref = oracle.forward(x[-34:], tr, suh, svh, k, cb, mode=1)
-    force(monkeypatch, r, 2)
-    check(run(lin, x).cpu().numpy()[-34:], ref, TOL_MODE1_REL, TOL_MODE1_ULP, "2 splits")
+    force(monkeypatch, r, 3)
+    check(run(lin, x).cpu().numpy()[-34:], ref, TOL_MODE1_REL, TOL_MODE1_ULP, "3 splits")
     force(monkeypatch, r, 1)
     y = run(lin, x).cpu().numpy()
     check(y[-34:], ref, TOL_MODE1_REL, TOL_MODE1_ULP, "1 split")
@@ -46,7 +45,7 @@ def test_every_k_and_codebook(monkeypatch, k, cb, r):
 
 
 @pytest.mark.parametrize("rows", [17, 64, 65, 127, 129, 256, 257, 513])
-@pytest.mark.parametrize("n_in, n_out, splits", [(128, 128, 1), (256, 256, 1), (1152, 640, 3)])
+@pytest.mark.parametrize("n_in, n_out, splits", [(128, 128, 1), (256, 256, 1), (1280, 640, 3)])
 def test_rows_and_widths(monkeypatch, rows, n_in, n_out, splits):
     for r in (4, 8, 16):
         print(f"wide rows={rows} {n_in}x{n_out} r={r}", flush=True)
@@ -64,12 +63,13 @@ def test_rows_and_widths(monkeypatch, rows, n_in, n_out, splits):
 @pytest.mark.parametrize("splits", [1, 3])
 def test_dtypes_bias_and_group(monkeypatch, dtype, bias, splits):
     """Every output form, through a group whose members end in a half pair: equal
-    to the members alone bit for bit (the same K-ranges)."""
+    to the members alone bit for bit (the same K-ranges: 14 steps, 3 splits of 4, 5
+    and 5)."""
     import mlxl3_amd
     import torch
 
-    made = [make_layer(6000 + i, 512, n_out, 3, 1, bias=bias) for i, n_out in enumerate((384, 128, 256))]
-    x = synth.activations(7, 1, 100, 512)
+    made = [make_layer(6000 + i, 896, n_out, 3, 1, bias=bias) for i, n_out in enumerate((384, 128, 256))]
+    x = synth.activations(7, 1, 100, 896)
     t = torch.from_numpy(x).cuda().to({"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}[dtype])
     force(monkeypatch, 8, splits)
     ys = mlxl3_amd.Exl3Group([m[0] for m in made]).forward(t)
@@ -87,6 +87,56 @@ def test_dtypes_bias_and_group(monkeypatch, dtype, bias, splits):
         # 2 ulp of the f16 result, one more of the last rounded format
         tol = 3 * ulp_of(np.abs(want).max(), dtype == "bf16")
         assert np.abs(got - want).max() <= tol, (dtype, bias, np.abs(got - want).max(), tol)
+
+
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("r", [4, 8, 16])
+@pytest.mark.parametrize("k,cb", [(3, 1), (4, 0), (5, 2), (8, 0)])
+def test_repeat_calls_bit_identical(monkeypatch, k, cb, r, splits):
+    """The loop keeps the wait states between its inline-assembly decode and the MFMAs,
+    and its counted waits for the copies, by hand: an error of that kind shows as
+    outputs that change between calls.  30 calls, two inputs in turn on one workspace
+    (what a call reads too early is the other input's), each equal to its input's first
+    result bit for bit."""
+    import torch
+
+    print(f"wide repeat k={k} cb={cb} r={r} splits={splits}", flush=True)
+    lin, _ = make_layer(7100 + k, 2816, 1152, k, cb)  # 44 steps: 14, 15, 15
+    force(monkeypatch, r, splits)
+    rows = 32 * r + 5
+    xs = [torch.from_numpy(synth.activations(70 + i, rows, rows, 2816)).cuda() for i in range(2)]
+    ws = torch.zeros(lin.workspace_bytes(rows), dtype=torch.uint8, device="cuda")
+    want = [lin.forward(x, workspace=ws).clone() for x in xs]
+    assert not torch.equal(want[0], want[1])
+    outs = [lin.forward(xs[i % 2], workspace=ws) for i in range(30)]
+    torch.cuda.synchronize()
+    for i, y in enumerate(outs):
+        assert torch.equal(y.view(torch.int16), want[i % 2].view(torch.int16)), i
+
+
+def test_unaligned_trellis_takes_the_producer_consumer_kernel(monkeypatch):
+    """The copies of the wide loop are 16 bytes wide: a trellis 8 bytes past that
+    alignment runs the other kernel, also where the wide one is forced, and gives its
+    bits."""
+    import mlxl3_amd
+    import torch
+
+    lin, (tr, suh, svh, _) = make_layer(7200, 2048, 384, 4, 0)
+    buf = torch.empty(lin.trellis.numel() + 4, dtype=torch.int16, device="cuda")[4:]
+    off = buf.view(lin.trellis.shape).copy_(lin.trellis)
+    assert off.data_ptr() % 16 == 8
+    moved = mlxl3_amd.Exl3Linear(off, lin.suh, lin.svh, None, 4, 0)
+    x = synth.activations(71, 1, 150, 2048)
+    monkeypatch.setenv("EXL3_QMM_SPLITS", "1")  # no partials, as the wide launch would have
+    monkeypatch.setenv("EXL3_WIDE", "0")
+    want, least = run(lin, x), lin.workspace_bytes(150)
+    monkeypatch.setenv("EXL3_WIDE", "1")
+    monkeypatch.setenv("EXL3_WIDE_TILE", "0")
+    monkeypatch.setenv("EXL3_WIDE_SPLITS", "8")
+    assert moved.workspace_bytes(150) == least < lin.workspace_bytes(150)
+    y = run(moved, x)
+    assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+    check(y.cpu().numpy(), oracle.forward(x, tr, suh, svh, 4, 0, mode=1), TOL_MODE1_REL, TOL_MODE1_ULP, "unaligned")
 
 
 def test_workspace_between_the_two_needs(monkeypatch):
@@ -189,6 +239,7 @@ def test_moe_wide_rows(monkeypatch, rows, gelu, score):
     import test_gpu_moe as m
 
     monkeypatch.setenv("EXL3_MOE_WIDE", "1")
+    monkeypatch.setenv("EXL3_MOE_GROUPED", "1")  # up to 64 slots too
     print(f"moe wide rows={rows} gelu={gelu} {score}", flush=True)
     layer, x, _, sc = m.case(384, 256, 3, 2, rows, 3, 720)
     sel = np.tile(np.array([[1, 2]], np.uint32), (rows, 1))
@@ -208,6 +259,12 @@ def test_moe_wide_rows(monkeypatch, rows, gelu, score):
     # the grouped kernel is held to the oracle by test_gpu_moe.py; both sum the same
     # products in the same order and differ by the epilogues' f32 sums
     m.check(y, other, "vs the 64-row blocks")
+    pick = sorted({min(1, rows - 1), rows // 2, rows - 1} - ({0} if rows > 1 else set()))
+    pick = [r for r in pick if (sel[r] < 3).all()]
+    if pick:
+        ref = oracle.moe_forward(x[pick], sel[pick], sc[pick].astype(score), *layer, 3, 0,
+                                 **(dict(activation="gelu", logical_hidden=200) if gelu else {}))
+        m.check(y[pick], ref, "rows of the oracle")
 
 
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16", "float32"])
@@ -227,6 +284,51 @@ def test_moe_wide_unaligned_input(monkeypatch, dtype):
     assert buf.data_ptr() % 16 != 0
     a, b = moe.forward(t, sel, sc), moe.forward(buf, sel, sc)
     assert torch.equal(a.float(), b.float())
+
+
+@pytest.mark.parametrize("part", [0, 3])
+def test_moe_unaligned_trellis_keeps_the_64_row_blocks(monkeypatch, part):
+    """A gate/up or down bank 8 bytes past its 16-byte alignment runs the 64-row blocks,
+    also where the wide ones are forced, and gives their bits."""
+    import test_gpu_moe as m
+    import mlxl3_amd
+    import torch
+
+    layer, x, sel, sc = m.case(256, 128, 5, 2, 260, 3, 750)
+    bank = [m.dev(a) for a in layer]
+    args = (m.dev(x), m.dev(sel), m.dev(sc))
+    monkeypatch.setenv("EXL3_MOE_WIDE", "0")
+    want = mlxl3_amd.Exl3SwitchGlu(*bank, top_k=2, k=3, cb=0).forward(*args)
+    buf = torch.empty(bank[part].numel() + 4, dtype=torch.int16, device="cuda")[4:]
+    bank[part] = buf.view(bank[part].shape).copy_(bank[part])
+    assert bank[part].data_ptr() % 16 == 8
+    monkeypatch.setenv("EXL3_MOE_WIDE", "1")
+    y = mlxl3_amd.Exl3SwitchGlu(*bank, top_k=2, k=3, cb=0).forward(*args)
+    assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("k,cb,gelu", [(3, 0, False), (4, 1, True), (6, 2, False), (8, 0, True)])
+def test_moe_wide_repeat_calls_bit_identical(monkeypatch, k, cb, gelu):
+    """test_repeat_calls_bit_identical for the expert form: 20 calls, two inputs and
+    routings in turn on one operator."""
+    import test_gpu_moe as m
+    import torch
+
+    print(f"moe wide repeat k={k} cb={cb} gelu={gelu}", flush=True)
+    monkeypatch.setenv("EXL3_MOE_WIDE", "1")
+    layer, _, _, _ = m.case(1152, 640, 6, 2, 4, k, 780)
+    moe = m.make_moe(layer, 2, k, cb, activation="gelu" if gelu else "silu")
+    ins = []
+    for i in range(2):
+        sel = routes_of([161, 37 + 3 * i, 160, 16, 200 - 3 * i, 2], 2, 781 + i)
+        _, sc = synth.moe_routes(783, i, sel.shape[0], 6, 2)
+        ins.append((m.dev(synth.activations(782, i, sel.shape[0], 1152)), m.dev(sel), m.dev(sc)))
+    want = [moe.forward(*a).clone() for a in ins]
+    assert not torch.equal(want[0], want[1])
+    outs = [moe.forward(*ins[i % 2]) for i in range(20)]
+    torch.cuda.synchronize()
+    for i, y in enumerate(outs):
+        assert torch.equal(y.view(torch.int16), want[i % 2].view(torch.int16)), i
 
 
 def routes_of(counts, top_k, seed, idle=0):
