@@ -1,9 +1,10 @@
 // MoE SwitchGLU entry points (Exl3SwitchGlu, native/src/moe.rs:611-1085):
 // validation as switch_glu_layout (native/src/contracts.rs:4-28) and
-// Exl3SwitchGlu::new (moe.rs:835-886), workspace layout, and the four
-// launches of the grouped expert path (route plan with the gather of the
-// gate/up inputs, gate/up QMM with the fused SwiGLU glue, down QMM with the
-// fused per-slot finish, top-k sum).
+// Exl3SwitchGlu::new (moe.rs:835-886), workspace layout, and the launches of
+// the grouped expert path: route plan with the gather of the gate/up inputs,
+// gate/up QMM with the fused SwiGLU glue, down QMM with the fused per-slot
+// finish, top-k sum; or, for many rows per expert, gate/up QMM, glue and down QMM
+// of exl3_moe_wide.hpp in place of the two (both where the device chooses).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -108,6 +109,12 @@ int moe_splits(const exl3_moe* h, int64_t slots, int block_rows, int k_in, int c
 //   K = 3, 4 1.6-1.8 1.09   1.9-2.0 0.93 even, 1.04 uneven   2.0-2.1 0.92   more 0.89
 //   K = 5, 6 1.5-1.7 0.98   1.7-1.8 0.95   1.9-2.0 0.85   more 0.80
 //   K = 8    0.87 at worst, so always
+// and, where that holds, by the gate/up workgroups per 512 (two on every CU): K <= 4 0.2-0.5
+// 0.94 to 1.03, 0.5-1 0.77 to 0.89, 1-1.25 1.07, 1.25-2 0.89 to 0.96, more 0.92 to 1.0; K = 5,
+// 6 below 0.3 0.89 to 0.98, else 0.73 to 0.96.  Two launches that find no blocks take 4 to
+// 6 us (9 in a trace), so the host leaves launches of less than half a round (0.3 of one
+// at K = 5, 6) to moe_mm_kernel (16 experts top-8, 256 tokens, 2048 x 768, K = 3: 94.9 us, 100.8
+// wide), and at K <= 4 the device those of 1 to 1.25 rounds.
 // GELU, whose glue in a launch of its own costs more (its binary64 tanh), above 112
 // rows per expert: K <= 4 never (1.09 at 2.0-2.1, 1.00 above 2.2), K = 5, 6 from 2.0 on
 // (0.92 even, 0.98 uneven), K = 8 always.
@@ -134,6 +141,7 @@ MoeWideMode moe_wide_mode(const exl3_moe* h, int64_t slots) {
   const int64_t wgs = h->experts * blocks * (2 * h->hidden / 128), slots_cu = 512;  // two per CU
   const int64_t rounds = (wgs + slots_cu - 1) / slots_cu;
   if (rounds > 1 && 4 * wgs < 3 * rounds * slots_cu) return kMoeNarrow;
+  if (10 * wgs < (h->k <= 4 ? 5 : h->k < 8 ? 3 : 0) * slots_cu) return kMoeNarrow;
   return h->k == 8 ? kMoeWideOnly : kMoeByBlocks;
 }
 
@@ -448,6 +456,7 @@ int exl3_moe_forward(const exl3_moe* h, const void* x, int32_t x_type, int64_t r
   pp.block_rows = L.block_rows;
   pp.alt_rows = L.wide == kMoeByBlocks ? moe_wide_rows(h->k) : 0;
   pp.alt_tenths = moe_wide_tenths(h);
+  pp.alt_units = h->k <= 4 ? 2 * h->hidden / 128 : 0;
   MoeGatherParams gp;
   gp.x = x;
   gp.x_dtype = x_type;

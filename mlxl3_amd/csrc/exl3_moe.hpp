@@ -23,12 +23,15 @@
 //               scores: an f32 product, MLX's promotion), stored per slot;
 //   4. reduce:  y[row] = sum over top_k in slot order in f32, then f16 (f16
 //               scores) or kept f32 (f32 or bf16 scores).
+// For many rows per expert launches 2 and 3 may be exl3_moe_wide.hpp's instead; where
+// that depends on the routes, both pairs are launched and the plan's counts leave one
+// of them without blocks.
 // Small inputs (decode: a handful of slots) split K over several workgroups
 // whose f32 partials meet in the last arriving one (agent-scope relaxed
 // atomics, as in the QMV), which adds them in split order.  Each row's
 // arithmetic is independent of the other rows of its block, so the
 // (atomics-ordered) placement of slots inside an expert's run cannot change any
-// result.
+// result (the kernel, and with it the order of some sums, follows the block counts).
 #pragma once
 
 #include "exl3_device.hpp"
@@ -55,6 +58,8 @@ struct MoePlanParams {
   int block_rows;            // 16, 32 or 64; 128 or 160 for moe_wide_kernel alone
   int alt_rows, alt_tenths;  // 0, or: blocks of alt_rows (128 or 160) rows where those of
                              // block_rows are at least alt_tenths / 10 times as many
+  int alt_units;             // 0, or: not where alt_units workgroups per block are more than
+                             // 512 and less than 640 (one round of the chip and a bit)
 };
 
 // The route plan, run by one workgroup of NT threads: counting sort of the
@@ -111,7 +116,9 @@ __device__ __forceinline__ void moe_plan_block(const MoePlanParams& p) {
   __syncthreads();
   int all_b = 0, all_a = 0;  // the whole call's blocks of either size
   for (int w = 0; w < NT / 64; ++w) all_b += wsum[1][w], all_a += wsum[2][w];
-  const bool alt = p.alt_rows && 10 * all_b >= p.alt_tenths * all_a;  // uniform
+  const int alt_wgs = min(all_a, 640) * p.alt_units;
+  const bool alt = p.alt_rows && 10 * all_b >= p.alt_tenths * all_a &&
+                   !(alt_wgs > 512 && alt_wgs < 640);  // uniform
   const int block_rows = alt ? alt_rows : p.block_rows;
   if (alt) ib = ia, lb = la;
   int bc = 0, bb = 0;

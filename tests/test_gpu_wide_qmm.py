@@ -340,9 +340,10 @@ def routes_of(counts, top_k, seed, idle=0):
     return ids.reshape(-1, top_k).astype(np.uint32)
 
 
-# 16 experts, mean rows per expert above the 64 (GELU: 112) from which the host lets
-# the device choose; wide: blocks of 160 rows are at least 2 (K = 3, 4 with SiLU: 1.9, K
-# = 5, 6: 1.7) times fewer than blocks of 64
+# 16 experts, hidden 1024 (16 workgroups a block), mean rows per expert above the 64
+# (GELU: 112) from which the host lets the device choose; wide: blocks of 160 rows are at
+# least 2 (K = 3, 4 with SiLU: 1.9, K = 5, 6: 1.7) times fewer than blocks of 64, and, for K
+# <= 4, their workgroups are not 513 to 639
 CHOICES = [
     # counts, k, activation, idle slots, wide
     ([80] * 16, 1, "silu", 0, True),                  # 32 against 16 blocks
@@ -358,9 +359,14 @@ CHOICES = [
     ([1, 0, 1279] + [0] * 13, 3, "silu", 0, True),    # 21 against 9, idle experts
     ([1, 0, 1279] + [0] * 13, 6, "silu", 16, True),   # ids outside the bank
     ([60] * 12 + [200] * 4, 6, "silu", 0, False),     # 28 against 20: 1.4
+    ([320] * 16, 4, "silu", 0, True),                 # 80 against 32: 512 workgroups
+    ([320] * 15 + [322], 4, "silu", 0, False),        # 81 against 33: 528
+    ([322] * 15 + [320], 5, "silu", 0, True),         # 95 against 47
+    ([322] * 7 + [320] * 9, 4, "silu", 0, False),     # 87 against 39: 624
+    ([322] * 8 + [320] * 8, 4, "silu", 0, True),      # 88 against 40: 640
     ([120] * 16, 4, "gelu", 0, False),                # GELU banks of K <= 4 never
     ([120] * 16, 5, "gelu", 0, True),
-    ([128] * 15 + [64], 6, "gelu", 0, False),       # 31 against 16 < 2
+    ([128] * 15 + [64], 6, "gelu", 0, False),         # 31 against 16 < 2
     ([30, 130] * 8, 8, "silu", 0, None),              # K = 8: always, nothing to choose
 ]
 
@@ -375,10 +381,10 @@ def test_moe_block_choice_follows_the_routes(monkeypatch, case_id):
 
     counts, k, act, idle, wide = CHOICES[case_id]
     print(f"moe choice {case_id} k={k} {act}", flush=True)
-    layer, _, _, _ = m.case(256, 128, 16, 2, 4, k, 760)
+    layer, _, _, _ = m.case(1024, 1024, 16, 2, 4, k, 760)
     sel = routes_of(counts, 2, 761 + case_id, idle)
     rows = sel.shape[0]
-    x = synth.activations(762, case_id, rows, 256)
+    x = synth.activations(762, case_id, rows, 1024)
     _, sc = synth.moe_routes(763, 1, rows, 16, 2)
     moe = m.make_moe(layer, 2, k, 0, activation=act)
     y = m.run(moe, x, sel, sc)
@@ -388,9 +394,7 @@ def test_moe_block_choice_follows_the_routes(monkeypatch, case_id):
     assert routed == sum(counts)
     if wide is not None:
         assert (narrow_blocks, wide_blocks) == ((0, bw) if wide else (b64, 0))
-    pick = np.arange(case_id % 5, rows, 11)
-    inside = (sel[pick] < 16).all(1)
-    pick = pick[inside]
+    pick = np.arange(rows)[(sel < 16).all(1)][case_id % 5::rows // 6]
     ref = oracle.moe_forward(x[pick], sel[pick], sc[pick], *layer, k, 0, activation=act)
     m.check(y[pick], ref, f"choice {case_id}")
     # two outputs that may each be TOL away from the oracle are at most twice that apart
@@ -402,18 +406,34 @@ def test_moe_block_choice_follows_the_routes(monkeypatch, case_id):
         assert np.abs(gap).max() <= 2 * m.TOL_RMS * rms, (case_id, forced)
 
 
+@pytest.mark.parametrize("k,hidden,may", [(4, 896, False), (4, 1024, True), (6, 512, False), (6, 640, True)])
+def test_moe_small_launches_keep_the_64_row_blocks(monkeypatch, k, hidden, may):
+    """Less than half a round of gate/up workgroups (16 experts of one block, hidden / 64 a
+    block, 512 a round; at K = 5, 6 0.3 of one) stays with 64-row blocks whatever the routes."""
+    import test_gpu_moe as m
+    import torch
+
+    layer, _, _, _ = m.case(1024, hidden, 16, 2, 4, k, 790)
+    sel = routes_of([80] * 16, 2, 791)
+    x = synth.activations(792, 1, sel.shape[0], 1024)
+    _, sc = synth.moe_routes(793, 1, sel.shape[0], 16, 2)
+    moe = m.make_moe(layer, 2, k, 0)
+    m.run(moe, x, sel, sc)
+    assert moe._ws.buf[65536:65536 + 12].view(torch.int32).tolist() == ([0, 1280, 16] if may else [32, 1280, 0])
+
+
 def test_moe_choice_alternates_on_one_workspace():
     """Even and uneven routes in turn on one operator (one workspace): each call equals
     its first result bit for bit, so neither kernel reads what the other left."""
     import test_gpu_moe as m
     import torch
 
-    layer, _, _, _ = m.case(512, 256, 16, 2, 4, 4, 770)
+    layer, _, _, _ = m.case(1024, 1024, 16, 2, 4, 4, 770)
     moe = m.make_moe(layer, 2, 4, 0)
     ins = []
     for i, counts in enumerate(([80] * 16, [30, 130, 30, 90] * 4, [30, 120] * 8)):
         sel = routes_of(counts, 2, 771 + i)
-        x = synth.activations(772, i, sel.shape[0], 512)
+        x = synth.activations(772, i, sel.shape[0], 1024)
         _, sc = synth.moe_routes(773, i, sel.shape[0], 16, 2)
         ins.append((m.dev(x), m.dev(sel), m.dev(sc)))
     want = [moe.forward(*a).clone() for a in ins]
