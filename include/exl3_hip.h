@@ -26,7 +26,9 @@
  * its first use (exl3_workspace_init does that on a stream); every call leaves
  * it reusable by any entry point (its first 64 KiB hold counters that every
  * call leaves at zero).  Calls that share one workspace must not run
- * concurrently.
+ * concurrently.  A QMM (rows > 16) may also run in somewhat less, with another
+ * K-split: results are equal bit for bit for workspaces of at least
+ * *_workspace_bytes, whatever their size.
  *
  * Threading: handles are immutable after creation and may be used from any
  * thread; error messages are per thread.
@@ -126,8 +128,10 @@ int exl3_linear_forward_noalloc(const exl3_linear* handle, const void* x, int32_
  * same input width, K and codebook applied to one x (q/k/v, gate/up); ys[i]
  * receives parts[i]'s output in exl3_linear_output_dtype(parts[i], x_type)
  * (x's dtype; f32 for a biased member under bf16 activations).  One launch covers every member's
- * column blocks (rows <= 16), or one prologue launch and one QMM launch (rows
- * > 16); each member's output is bit-identical to its own exl3_linear_forward.
+ * column blocks (rows <= 16), or one prologue launch and one QMM (rows > 16).
+ * Each member's output is bit-identical to its own exl3_linear_forward where
+ * both split K alike; the splits follow the launch's total width, so other
+ * members may differ from it in the order of their f32 sums (2 f16 ulp).
  * Workspace: exl3_group_workspace_bytes. */
 size_t exl3_group_workspace_bytes(const exl3_linear* const* parts, int32_t count, int64_t rows);
 int exl3_group_forward(const exl3_linear* const* parts, int32_t count, const void* x,
@@ -151,7 +155,8 @@ int exl3_geglu(const uint16_t* gate, const uint16_t* up, uint16_t* out, int64_t 
  * gate/up, Array::swiglu, down Exl3Linear::forward): y[rows][down.out] =
  * down(swiglu(gate(x), up(x))), f16 x and y; gate and up share in, out, K and
  * codebook, down.in = gate.out.  The SwiGLU (and, for rows > 16, the down
- * projection's input prologue) runs in the epilogue of the (gate, up) launch;
+ * projection's input prologue) runs in the epilogue of the (gate, up) launch
+ * (rows <= 16) or in one launch after it;
  * the result is bit-identical to exl3_group_forward + exl3_swiglu +
  * exl3_linear_forward.  Workspace: exl3_mlp_workspace_bytes. */
 size_t exl3_mlp_workspace_bytes(const exl3_linear* gate, const exl3_linear* up,

@@ -332,7 +332,8 @@ static size_t qmm_partial_bytes(const QmmShape& sh, int out) {
 // launch; fitted to a sweep of every tile and split count over seven shapes x 32 to
 // 4096 rows at K = 4 (one box), where it is within 3 % of the fastest measured but
 // where the partials of more splits would pass the allocation-free entry point's
-// budget.  Against the producer/consumer kernel there (us, calls): 4096x28672 rows
+// budget.  Against the producer/consumer kernel there (us, calls; that kernel before its
+// epilogue by MFMA, plan_wide has the present comparison): 4096x28672 rows
 // 384/512/1024/2048 147/142/285/521 -> 112/117/228/461, 14336x4096 rows
 // 768/2048/4096 126/259/524 -> 111/247/442, 27648x5120 rows 384/512/1024
 // 167/175/339 -> 138/158/287, 5120x7168 rows 2048/4096 185/353 -> 148/289, 4096x14336

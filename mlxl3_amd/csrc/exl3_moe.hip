@@ -108,7 +108,7 @@ int moe_splits(const exl3_moe* h, int64_t slots, int block_rows, int k_in, int c
 //   K <= 2   1.6-1.8 1.10-1.18   1.9-2.0 1.02   2.0-2.1 0.98   2.1-2.2 0.94   more 0.89
 //   K = 3, 4 1.6-1.8 1.09   1.9-2.0 0.93 even, 1.04 uneven   2.0-2.1 0.92   more 0.89
 //   K = 5, 6 1.5-1.7 0.98   1.7-1.8 0.95   1.9-2.0 0.85   more 0.80
-//   K = 8    0.87 at worst, so always
+//   K = 8    0.70 even, 0.75 uneven, 1.0 at worst, so always
 // and, where that holds, by the gate/up workgroups per 512 (two on every CU): K <= 4 0.2-0.5
 // 0.94 to 1.03, 0.5-1 0.77 to 0.89, 1-1.25 1.07, 1.25-2 0.89 to 0.96, more 0.92 to 1.0; K = 5,
 // 6 below 0.3 0.89 to 0.98, else 0.73 to 0.96.  Two launches that find no blocks take 4 to

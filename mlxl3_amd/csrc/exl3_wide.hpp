@@ -21,9 +21,9 @@
 // per MFMA: n=2 16.8, 4 25.0, 5 28.8), the decode of K = 4 adds 4.5 per MFMA at R =
 // 8 and 2.25 at R = 16; past that the card's power: the same loop with the decode
 // left out (timing only) runs its MFMAs at ~1260 TFLOP/s and a lower clock.
-// Measured, 4096 -> 14336, K = 4 (kernel, us and TFLOP/s): 512 rows, R = 8, 77 / 780
-// (producer/consumer kernel 80-86), 2048 rows, R = 16, 241 / 997 (305 / 790).  Forms
-// that were no faster: 32x32x16 MFMAs with 64 columns per wave and two K halves (714
+// Measured, 4096 -> 14336, K = 4 (a call, us): 2048 rows, R = 16, 236 to 239 (1007 to 1019
+// TFLOP/s; the producer/consumer kernel 285); 512 rows, R = 8, 77 to 78, where that kernel
+// with the same epilogue takes 75 to 76 and keeps the launch.  Forms that were no faster: 32x32x16 MFMAs with 64 columns per wave and two K halves (714
 // TFLOP/s at 512 rows, fewer cycles at a lower clock), the same with one wave per
 // SIMD and 256 rows (878 at 2048 rows), trellis words read one step later.
 #pragma once
