@@ -190,6 +190,23 @@ def test_prologue_on_both_sides_of_the_rule(rows, dtype, off):
     assert np.abs(y - want).max() <= 3 * ulp_of(np.abs(want).max(), dtype == "bf16")
 
 
+@pytest.mark.parametrize("n_in,hidden,rows", [(1024, 3584, 40), (1024, 3584, 300), (768, 4096, 700)])
+def test_mlp_equals_its_parts_at_split_launches(n_in, hidden, rows):
+    """Shapes whose launches split K under the default rules: the fused MLP, whose
+    workspace leaves its down projection other room than the linear's own, still equals
+    the group, the SwiGLU and the linear bit for bit."""
+    import mlxl3_amd
+    import torch
+    import test_gpu_group as g
+
+    _, parts, _ = g.mlp_case(n_in, hidden, 4, 0)
+    x = torch.from_numpy(synth.activations(11, rows, rows, n_in)).cuda()
+    down = parts[2]
+    assert down.workspace_bytes(rows) > 65536 + 2 * rows * hidden + 255  # partials: it splits
+    y, other = mlxl3_amd.Exl3Mlp(*parts).forward(x), g.unfused(parts, x)
+    assert torch.equal(y.view(torch.int16), other.view(torch.int16))
+
+
 @pytest.mark.parametrize("rows", [2032, 2033])
 @pytest.mark.parametrize("off", [0, 1])
 def test_swiglu_edge_on_both_sides_of_the_rule(rows, off):
@@ -441,6 +458,38 @@ def test_moe_choice_alternates_on_one_workspace():
     torch.cuda.synchronize()
     for i, y in enumerate(outs):
         assert torch.equal(y.view(torch.int16), want[i % 3].view(torch.int16)), i
+
+
+def test_moe_choice_under_capture():
+    """The choice is made by each replay: one captured call, its routes rewritten between
+    replays so that either kernel has the blocks, equals the eager call every time."""
+    import test_gpu_moe as m
+    import torch
+
+    layer, _, _, _ = m.case(1024, 1024, 16, 2, 4, 4, 770)
+    moe = m.make_moe(layer, 2, 4, 0)
+    routes = [m.dev(routes_of(c, 2, 775 + i)).to(torch.int32) for i, c in enumerate(([80] * 16, [30, 130, 60, 100] * 4))]
+    rows = routes[0].shape[0]
+    x = m.dev(synth.activations(776, 1, rows, 1024))
+    sc = m.dev(synth.moe_routes(777, 1, rows, 16, 2)[1])
+    want = [moe.forward(x, sel, sc).clone() for sel in routes]
+    assert not torch.equal(want[0], want[1])
+    sel = routes[0].clone()
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        moe.forward(x, sel, sc)
+    torch.cuda.current_stream().wait_stream(s)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = moe.forward(x, sel, sc)
+    for i in (0, 1, 1, 0, 1, 0):
+        sel.copy_(routes[i])
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.int16), want[i].view(torch.int16)), i
+        wide = int(moe._ws.buf[65536 + 8:65536 + 12].view(torch.int32))
+        assert (wide > 0) == (i == 0)
 
 
 @pytest.mark.parametrize("experts", [3840, 4096])
