@@ -492,14 +492,15 @@ static size_t wide_partials(const Group& g, int64_t rows, const WideLaunch& w) {
 // (whose model leaves out ~6 us of ring fill and epilogue).  That model's step times
 // were fitted at K = 4 with an earlier epilogue and price some launches too high; they
 // stay as they are where they choose that kernel's own shape, and are corrected here
-// (us a call with rotated weights, that kernel / this one, 11850 random shapes x rows
-// x K: of 5454 calls taken at its full price 160 lost more than 2 % against its earlier
-// form, up to 11 %; 23 of 4748 are left, and 34 of 3572 in another 8950, most of them
-// inputs of 13000 and more):
-//   * one round of MB = 4 tiles at K <= 4 against one 128 x 256 split here, which
-//     decodes every weight twice as often, 0.86: 5120 x 27648 rows 172 K = 3 87.6 / 94.4,
-//     rows 152 K = 1 83.9 / 89.3, 8960 x 28416 rows 131 K = 3 143.6 / 156.2.  At K >= 5
-//     that kernel's producers are the slower part and the model holds;
+// (us a call with rotated weights, that kernel / this one; of 31630 random shapes x rows
+// x K, 14422 were taken at its full price, 591 of them more than 2 %, up to 11 %, slower
+// than its earlier form; now 12207 are, 52 of them slower):
+//   * MB = 4 tiles never give way to unsplit 128 x 256 tiles at K <= 4, which decode
+//     every weight twice as often: 5120 x 27648 rows 172 K = 3 87.6 / 94.4, rows 152 K = 1
+//     83.9 / 89.3, rows 604 K = 3 260 / 286, 8960 x 28416 rows 131 K = 3 143.6 / 156.2; nor, in
+//     one round, for inputs of 12800 and more at K = 5 to 7 (26112 x 27520 rows 144 K = 5 413
+//     / 437), where the step time here grows.  Elsewhere at K >= 5 that kernel's
+//     producers are the slower part and the model holds;
 //   * up to 64 rows in one round of MB = 1 tiles against 128 x 256, 0.9: 5120 x 27648 rows 32 K = 4
 //     51.4 / 53.9, rows 35 K = 1 50.6 / 57.0, K = 6 56.5 / 61.9;
 //   * two MB = 1 workgroups share a CU, which the model leaves out past 256 of them,
@@ -513,11 +514,10 @@ static void plan_wide(const Group& g, int64_t rows, size_t budget, QmmPlan& p) {
   const bool one_round = (int64_t)p.q.mtiles * (g.total_out / 128) * p.q.splits <= 256;
   const bool tile128 = p.w.kind == 1;
   double price = 1.0;
-  if (p.q.mb == 1)
-    price = !one_round ? 0.75 : tile128 && rows <= 64 ? 0.9 : 1.0;
-  else if (p.q.mb == 4 && one_round && tile128 && p.w.splits == 1 && g.k <= 4)
-    price = 0.86;
-  p.wide = p.forced_wide || ((p.w.splits == 1 || p.q.cost >= 20000.0) &&
+  if (p.q.mb == 1) price = !one_round ? 0.75 : tile128 && rows <= 64 ? 0.9 : 1.0;
+  const bool twice = p.q.mb == 4 && tile128 && p.w.splits == 1 &&
+                     (g.k <= 4 || (g.k < 8 && one_round && g.in >= 12800));
+  p.wide = p.forced_wide || (!twice && (p.w.splits == 1 || p.q.cost >= 20000.0) &&
                              p.w.cost < price * p.q.cost + 6000.0);
 }
 
